@@ -237,7 +237,7 @@ private:
   bool force_stream0_ = false;  // level 0 streamed for every domain (projection solves)
   bool zg0_ = false;            // the stages being launched apply ZG at level 0
   // levels run as fused tile passes (smoothing counts with a tiled pass)
-  bool tiled() const { return tile_pass_ok(prm_.nu_pre) && tile_pass_ok(prm_.nu_post); }
+  bool tiled() const { return prm_.nu_pre <= kNuPass && prm_.nu_post <= kNuPass; }
   // level l of a domain of this shape may run as row-streamed passes (wide
   // and large levels) ...
   bool stream_eligible(const BGeom &G, int l) const;

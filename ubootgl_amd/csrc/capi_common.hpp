@@ -48,10 +48,6 @@ inline int check_launch() {
 
 inline size_t align_up(size_t n, size_t a = 256) { return (n + a - 1) / a * a; }
 
-// levels with at least this many cells run the row-streamed level kernels
-// (below, a level has too few strip x row-block units to fill the chip and
-// the LDS tiles are faster)
-constexpr size_t kFuseMinCells = (size_t)1 << 22;
 // the single-workgroup LDS V-cycle starts at the first level with at most
 // this many cells (one CU's lanes do all of its work, so larger levels run
 // faster as tiles spread over the chip; measured: starting at 8192 cells
@@ -219,20 +215,20 @@ struct ubg_mg {
   }
 
   // Whether solve_level(l) (l > 0: zero initial guess, no ZG) reads its p
-  // before writing it.  The LDS coarse V-cycle and the tile pre pass do not,
-  // so the restriction above may leave that p as it is instead of zeroing it
+  // before writing it.  The LDS coarse V-cycle and the pre pass do not, so
+  // the restriction above may leave that p as it is instead of zeroing it
   // (the branches of solve_level decide alike).
   bool reads_zero_p(int l) {
-    const size_t n = (size_t)lv[l].w * lv[l].h;
     if (l == levels - 2) return true; // sweeps on the coarsest solved level
-    if (n <= kCoarseMaxCells && coarse_fits_lds(lv.data(), l, levels)) return false;
-    if (n < kFuseMinCells && tile_pass_ok(prm.nu_pre) && tile_pass_ok(prm.nu_post)) return false;
-    return true;
+    if ((size_t)lv[l].w * lv[l].h <= kCoarseMaxCells && coarse_fits_lds(lv.data(), l, levels))
+      return false;
+    return prm.nu_pre > kNuPass; // sweeps before the pre pass
   }
 
-  // MG::solveLevel (pressure_solver.cpp:201-248).  A level costs two fused
-  // passes: (pre-smoothing, residual, restriction) and (prolongation,
-  // correction, post-smoothing); setZeroGradientBC happens inside them.
+  // MG::solveLevel (pressure_solver.cpp:201-248).  A level costs two
+  // launches: (pre-smoothing, residual, restriction) and (prolongation,
+  // correction, post-smoothing), setZeroGradientBC inside them; smoothing
+  // counts above kNuPass take the rest as single sweeps.
   void solve_level(int l, float h, bool zg) {
     const bool z = zg && l == 0;
     if (l == levels - 2) {
@@ -246,35 +242,16 @@ struct ubg_mg {
       return;
     }
     Level &L = lv[l], &C = lv[l + 1];
-    if ((size_t)L.w * L.h < kFuseMinCells) {
-      float hc = h * (L.w - 1.0f) / (C.w - 1.0f); // pressure_solver.cpp:229
-      if (!z && tile_pass_ok(prm.nu_pre) && tile_pass_ok(prm.nu_post)) {
-        // small level: two LDS-tiled launches instead of 2 + nu_pre + nu_post
-        launch_tile_pre(L, C, prm.nu_pre, h, prm.alpha, l > 0, reads_zero_p(l + 1), stream);
-        solve_level(l + 1, hc, false);
-        launch_tile_post(L, C, prm.nu_post, h, prm.alpha, stream);
-        return;
-      }
-      sweeps(l, prm.nu_pre, h, z);
-      launch_residual_restrict(L, C, h, stream);
-      solve_level(l + 1, hc, false);
-      launch_prolong_correct(L, C, stream);
-      if (z) launch_zero_gradient(L.p, L.w, L.h, stream);
-      sweeps(l, prm.nu_post, h, z);
-      return;
-    }
-    // the last pre-smoothing sweep and the first post-smoothing sweep ride in
-    // the grid-transfer passes
-    const int pre_fused = std::min(prm.nu_pre, 1);
-    sweeps(l, prm.nu_pre - pre_fused, h, z);
+    const int pre = std::min(prm.nu_pre, kNuPass), post = std::min(prm.nu_post, kNuPass);
+    sweeps(l, prm.nu_pre - pre, h, z);
     timed(UBG_TIMER_L0_PRE, l, [&] {
-      launch_presmooth_restrict(L, C, pre_fused, h, prm.alpha, z, reads_zero_p(l + 1), stream);
+      launch_level_pre(L, C, pre, h, prm.alpha, l > 0 && prm.nu_pre <= kNuPass, z,
+                       reads_zero_p(l + 1), stream);
     });
-    float hc = h * (L.w - 1.0f) / (C.w - 1.0f); // pressure_solver.cpp:229
-    solve_level(l + 1, hc, false);
-    const int post_fused = std::min(prm.nu_post, 1);
-    timed(UBG_TIMER_L0_POST, l, [&] { launch_prolong_postsmooth(L, C, post_fused, h, prm.alpha, z, stream); });
-    sweeps(l, prm.nu_post - post_fused, h, z);
+    solve_level(l + 1, h * (L.w - 1.0f) / (C.w - 1.0f), false); // pressure_solver.cpp:229
+    timed(UBG_TIMER_L0_POST, l,
+          [&] { launch_level_post(L, C, post, h, prm.alpha, z, stream); });
+    sweeps(l, prm.nu_post - post, h, z);
   }
 
   // coarse flags of levels 1..L-1 from the level-0 flag (updateFields)

@@ -85,26 +85,18 @@ void launch_coarsen(const uint8_t *ff, int wf, uint8_t *fc, int wc, int hc, hipS
 // setZeroGradientBC to the result.
 void launch_rbgs_fused(Level &L, float h, float alpha, bool zero_gradient, hipStream_t s);
 void launch_zero_gradient(float *p, int w, int h, hipStream_t s);
-// Row-pipelined level passes (ping-pong: read L.p, write L.p_alt, swap):
-//   ns (0 or 1) sweeps, then residual + restriction into C
-//   (C.f = restricted residual, C.p = 0 if zero_coarse, else C.p is left as
-//   it is for a coarse pass that does not read it);
-void launch_presmooth_restrict(Level &L, Level &C, int ns, float h, float alpha, bool zg,
-                               bool zero_coarse, hipStream_t s);
-//   prolongation of C.p + correction (+ZG), then ns (0 or 1) sweeps.
-void launch_prolong_postsmooth(Level &L, const Level &C, int ns, float h, float alpha, bool zg,
-                               hipStream_t s);
-// LDS-tiled level passes (mg_tile.hip) for levels below the streaming size:
-// nu sweeps + residual + restriction, and prolongation + correction + nu
-// sweeps, one launch each; both swap L.p / L.p_alt.  No zero-gradient BC.
-// zero_p: L.p is zero on entry (every level below the finest: the
-// restriction above zeroed it), so the pre pass does not read it;
-// zero_coarse: the pre pass zeroes C.p (else C.p is left as it is, for a
-// coarse pass that does not read it).
-bool tile_pass_ok(int nu);
-void launch_tile_pre(Level &L, Level &C, int nu, float h, float alpha, bool zero_p,
-                     bool zero_coarse, hipStream_t s);
-void launch_tile_post(Level &L, const Level &C, int nu, float h, float alpha, hipStream_t s);
+// Level passes (mg_regtile.hip; ping-pong: read L.p, write L.p_alt, swap) of
+// up to kNuPass sweeps:
+//   nu sweeps, residual, restriction into C.  zero_p: L.p is zero on entry
+//   and is not read; zero_coarse: C.p = 0 in the interior (else C.p is left
+//   as it is, for a coarse pass that does not read it);
+constexpr int kNuPass = 3;
+void launch_level_pre(Level &L, Level &C, int nu, float h, float alpha, bool zero_p, bool zg,
+                      bool zero_coarse, hipStream_t s);
+//   prolongation of C.p, correction, nu sweeps.
+// zg: setZeroGradientBC after every sweep and after the correction.
+void launch_level_post(Level &L, const Level &C, int nu, float h, float alpha, bool zg,
+                       hipStream_t s);
 void launch_residual(const Level &L, float h, hipStream_t s);
 void launch_residual_restrict(const Level &F, const Level &C, float h, hipStream_t s);
 void launch_prolong_correct(const Level &F, const Level &C, hipStream_t s);
