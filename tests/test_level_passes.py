@@ -64,3 +64,34 @@ def test_level_passes_bit_exact(gpu, W, H, nu, kind, alpha, zg):
         om.solve(want, f, flag, h, zg)
     np.testing.assert_array_equal(p, want)
     mg.close()
+
+
+# domains so elongated that the coarsest solved level is larger than the LDS
+# V-cycle's usual first level (4, 6 pairs of cells per thread), beside an
+# ordinary one and ones whose LDS levels have odd widths and one or two pairs
+@pytest.mark.parametrize("sizes", [[(2000, 16), (200, 100)], [(2980, 17), (16, 1700)],
+                                   [(75, 131), (139, 111), (33, 1000)]])
+def test_batch_lds_levels_match_single(gpu, sizes):
+    from ubootgl_amd.batch import Batch
+    g = np.random.default_rng(3)
+    b, want = Batch(sizes), []
+    for d, (W, H) in enumerate(sizes):
+        flag = flags(W, H, "noise", d)
+        flag[0] = flag[-1] = 1
+        flag[:, 0] = flag[:, -1] = 1
+        # pockets without a path to the ring would be singular
+        flag[1:-1, 1:-1] = np.where(g.random((H - 2, W - 2)) < 0.04, 0, 1)
+        f = (g.standard_normal((H, W)) * flag).astype(np.float32)
+        f[0] = f[-1] = 0
+        f[:, 0] = f[:, -1] = 0
+        b.set_domain(d, flag, f, 1.0 / W)
+        mg = U.MG(flag)
+        mg.ir_set_rhs(f)
+        mg.ir_set_guess(None)
+        mg.ir_solve(float(np.float32(1.0 / W)), tol=1e-5, raise_on_stall=False)
+        want.append(mg.ir_solution())
+        mg.close()
+    b.solve(tol=1e-5, raise_on_stall=False)
+    for d in range(len(sizes)):
+        np.testing.assert_array_equal(b.solution(d), want[d])
+    b.close()

@@ -397,6 +397,7 @@ __global__ void __launch_bounds__(TPB) kb_stream_pass(StageArgs a) {
 
 // the coarse levels of each domain in LDS, one workgroup per domain slot;
 // ia: index of p at the domain's first LDS level
+template <bool BIG>
 __global__ void __launch_bounds__(TPB_C) kb_coarse(StageArgs a, const CoarseArgs *cargs,
                                                    int nslots) {
   const int d = blockIdx.x;
@@ -404,7 +405,7 @@ __global__ void __launch_bounds__(TPB_C) kb_coarse(StageArgs a, const CoarseArgs
   const BDom &D = a.dom[d];
   if (!dom_active(D) || D.cfirst >= D.nlev) return;
   const BLev &L = a.lev[d * BMAXL + D.cfirst];
-  coarse_vcycle_body(cargs[d], L.f, L.p[a.ia[d]]);
+  coarse_vcycle_body<BIG>(cargs[d], L.f, L.p[a.ia[d]]);
 }
 
 __device__ __forceinline__ double wsum(double v) {
@@ -760,12 +761,13 @@ int BatchEngine::init(hipStream_t s, const ubg_params &prm, int vcycles_per_step
   UBG_HIP(hipMalloc((void **)&d_count_, sizeof(int)));
   UBG_HIP(hipHostMalloc((void **)&count_host_, sizeof(int), hipHostMallocDefault));
   *count_host_ = 0;
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute((const void *)kb_coarse, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)LDS_BUDGET);
-    attr = true;
-  }
+  static const bool attr_set = [] { // more than 64 KiB of LDS
+    for (auto k : {kb_coarse<false>, kb_coarse<true>})
+      (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)LDS_BUDGET);
+    return true;
+  }();
+  (void)attr_set;
   return UBG_OK;
 }
 
@@ -1000,6 +1002,7 @@ int BatchEngine::build_tables() {
   std::vector<BDom> dom(std::max<size_t>(n, 1));
   std::vector<CoarseArgs> ca(std::max<size_t>(n, 1));
   coarse_lds_ = 0;
+  coarse_big_ = false;
   lmax_ = 0;
   for (size_t s = 0; s < n; s++) {
     const BDomain &D = *all_[s];
@@ -1037,6 +1040,7 @@ int BatchEngine::build_tables() {
       a.h[k] = G.h[l];
       a.mask[k] = G.mask[l];
       a.hh[k] = D.hh[l];
+      a.ihsq[k] = 1.0f / D.hh[l] / D.hh[l];
     }
     a.nu_pre = prm_.nu_pre;
     a.nu_post = prm_.nu_post;
@@ -1044,6 +1048,7 @@ int BatchEngine::build_tables() {
     a.alpha = prm_.alpha;
     if (s < run_.size()) {
       coarse_lds_ = std::max(coarse_lds_, G.lds_bytes);
+      coarse_big_ = coarse_big_ || coarse_big(G.w[G.cfirst], G.h[G.cfirst]);
       lmax_ = std::max(lmax_, G.cfirst);
     }
   }
@@ -1411,7 +1416,7 @@ int BatchEngine::launch_stages(const std::vector<StageRec> &st, const uint8_t *d
       break;
     case ST_COARSE:
       if (!run_.empty())
-        hipLaunchKernelGGL(kb_coarse, dim3((unsigned)run_.size()), dim3(TPB_C), coarse_lds_,
+        hipLaunchKernelGGL((coarse_big_ ? kb_coarse<true> : kb_coarse<false>), dim3((unsigned)run_.size()), dim3(TPB_C), coarse_lds_,
                            stream_, a, (const CoarseArgs *)d_cargs_, (int)run_.size());
       break;
     case ST_UPDATE:

@@ -218,6 +218,7 @@ private:
   CoarseArgs *d_cargs_ = nullptr;
   size_t tab_cap_ = 0;
   size_t coarse_lds_ = 0;
+  bool coarse_big_ = false; // a member's first LDS level needs the larger variant
   // tile maps: per level sweep / rr / pc (running members), update (all):
   // prefix of tile counts over slots and tiles per row, in one int array
   std::vector<int> h_off_;

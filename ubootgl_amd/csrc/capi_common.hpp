@@ -3,6 +3,7 @@
 // the C ABI translation units.
 #pragma once
 
+#include "coarse_device.hpp"
 #include "ubg_internal.hpp"
 #include "../../include/ubg_c.h"
 
@@ -47,12 +48,6 @@ inline int check_launch() {
 }
 
 inline size_t align_up(size_t n, size_t a = 256) { return (n + a - 1) / a * a; }
-
-// the single-workgroup LDS V-cycle starts at the first level with at most
-// this many cells (one CU's lanes do all of its work, so larger levels run
-// faster as tiles spread over the chip; measured: starting at 8192 cells
-// slows the 4096x2048 step by ~2%)
-constexpr size_t kCoarseMaxCells = 4096;
 
 // A simple bump allocator over one hipMalloc.
 struct Pool {

@@ -12,11 +12,18 @@ constexpr int MAXL = 16;
 constexpr int TPB_C = 1024;
 constexpr int WAVES_C = TPB_C / 64;
 constexpr size_t LDS_BUDGET = 152 * 1024;
+// The single-workgroup LDS V-cycle starts at the first level with at most
+// this many cells: one CU does all of its work, so larger levels run faster as
+// tiles spread over the chip (128x64 and below in LDS at 3/3/5 sweeps: 32 us,
+// against 12.5 us from 64x32 and 12.6 us for the tiles of 128x64).
+constexpr size_t kCoarseMaxCells = 4096;
 
 struct CoarseArgs {
   int n; // levels first .. L-2
   int w[MAXL], h[MAXL];
   float hh[MAXL];
+  float ihsq[MAXL]; // 1 / h / h
+  float iw[MAXL];   // 1 / w
   int op[MAXL], of[MAXL], om[MAXL]; // LDS byte offsets of p, f, mask
   int orr;                           // residual scratch (first level's size)
   const uint8_t *mask[MAXL];
@@ -26,270 +33,415 @@ struct CoarseArgs {
   float alpha;
 };
 
-// 1024 threads as 16 waves x 64 lanes.  A level row with at most `count`
-// items (cells of a colour, cells, blocks) takes L lanes, L the smallest
-// power of two >= count (at most 64), so a wave holds G = 64 / L rows at
-// once: lane group g of wave ty starts at row offset G ty + g and steps by
-// 16 G.  On the narrow coarse levels this packs 2-8 consecutive rows into
-// one wave, so a level of few rows keeps few waves busy (and few per SIMD)
-// instead of one partly filled wave per row.
-struct RowGroups {
-  int lr;   // lane within the row group
-  int r0;   // first row offset (G * wave + group)
-  int step; // row step, 16 * G
-  int L;    // lanes per row
-};
-__device__ __forceinline__ RowGroups row_groups(int count) {
-  int lg = 6;
-  while (lg > 0 && (1 << (lg - 1)) >= count) lg--;
-  const int tx = threadIdx.x & 63;
-  const int ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  RowGroups r;
-  r.L = 1 << lg;
-  r.lr = tx & (r.L - 1);
-  r.r0 = (ty << (6 - lg)) + (tx >> lg);
-  r.step = WAVES_C << (6 - lg);
-  return r;
-}
-
-// A cell's smoothing constants, decoded once from its mask byte and f for
-// sweeps that update the same cell again and again.  smooth_rule performs
-// the operations of smooth() in the same order (the division by the count
-// as div_count does it), so the results are identical.
+// Threads own pairs of cells: thread t has pair t, t + 1024, ... of a level,
+// pair t being the cells 2t and 2t + 1 in row-major order -- one red
+// ((x + y) odd) and one black, neighbours in a row (or, at an odd width, two
+// ring cells of adjacent rows).  For a visit of the level the pair's p, f and
+// decoded smoothing rules stay in registers (the first level's for the whole
+// V-cycle).  LDS holds p for the neighbours, the red cells and the black ones
+// each in a plane of their own, entry i >> 1 for cell i: a colour reads only
+// the other plane, and a wave's lanes read consecutive words.  An update is
+// three LDS reads (its partner is a register) and one write.
+//
+// What bounds this kernel is latency and the instructions of one CU: about
+// 35 dependent colour phases and two grid transfers per pair of levels.
+// Measured on gfx950 (64x32 down to 16x8, 3/3/5 sweeps; 64x64 down to 8x8):
+// 12.4 and 19.7 us, against 15.2 and 27.4 us with one cell per
+// thread and phase in row-major LDS, whose transfers alone cost 3.2 us per
+// pair of levels (integer divisions, idle waves at work, two-way bank
+// conflicts in every phase).
+//
+// A cell's smoothing constants, decoded from its mask byte and f.  smooth_rule
+// performs the operations of smooth() (the division by the count as div_count
+// does it); the first two addends, W and E, are its outside and its partner
+// neighbour in either order, which rounds alike.
 struct CellRule {
-  int sw, se, ss, sn; // 0 / -1: the neighbour's value is kept, or +0 added
+  int so, sp, ss, sn; // 0 / -1: the neighbour's value is kept, or +0 added
   float inv, ns;      // RN(1 / s) and -s for the neighbour count s
   float F, fhh;       // own flag (0 / 1) and (f * h) * h
-  bool empty;         // s == 0: the quotient is +0
+  int some;           // 0 when s == 0 (the quotient is +0), else -1
 };
-__device__ __forceinline__ CellRule cell_rule(unsigned mk, float fv, float h) {
+__device__ __forceinline__ CellRule cell_rule(unsigned mk, bool out_west, float fv, float h) {
   CellRule c;
-  c.sw = -(int)((mk >> 1) & 1u);
-  c.se = -(int)((mk >> 2) & 1u);
+  const int sw = -(int)((mk >> 1) & 1u), se = -(int)((mk >> 2) & 1u);
+  c.so = out_west ? sw : se;
+  c.sp = out_west ? se : sw;
   c.ss = -(int)((mk >> 3) & 1u);
   c.sn = -(int)((mk >> 4) & 1u);
   const unsigned s = mk >> 5;
   const float pow2 = __int_as_float((int)((127u - (s >> 1)) << 23));
   c.inv = (s == 3u) ? (1.0f / 3.0f) : pow2;
   c.ns = -(float)s;
-  c.empty = s == 0u;
+  c.some = s == 0u ? 0 : -1;
   c.F = (float)(mk & MK_SELF);
   c.fhh = fv * h * h;
   return c;
 }
-__device__ __forceinline__ float smooth_rule(float pc, float pw, float pe, float ps, float pn,
+__device__ __forceinline__ float keep(int sel, float v) {
+  return __int_as_float(__float_as_int(v) & sel);
+}
+__device__ __forceinline__ float pick(int sel, float v, float c) {
+  return __int_as_float((__float_as_int(v) & sel) | (__float_as_int(c) & ~sel));
+}
+__device__ __forceinline__ float smooth_rule(float pc, float po, float pp, float ps, float pn,
                                              const CellRule &c, float alpha) {
   float val = 0.0f;
-  val += __int_as_float(__float_as_int(pw) & c.sw);
-  val += __int_as_float(__float_as_int(pe) & c.se);
-  val += __int_as_float(__float_as_int(ps) & c.ss);
-  val += __int_as_float(__float_as_int(pn) & c.sn);
+  val += keep(c.so, po);
+  val += keep(c.sp, pp);
+  val += keep(c.ss, ps);
+  val += keep(c.sn, pn);
   val += c.fhh;
   const float q = val * c.inv;
   const float r = fmaf(c.ns, q, val);
   const float q2 = fmaf(r, c.inv, q);
-  val = c.empty ? 0.0f : q2;
+  val = keep(c.some, q2);
   return c.F * (alpha * val + (1.0f - alpha) * pc);
 }
-
-// nu red+black sweeps of a w x h level in LDS.  A row's cells of a colour
-// are at most (w - 1) / 2; rows of one lane group share the colour parity
-// (their offsets differ by multiples of 16).  When the lane groups cover
-// every interior row and every cell of a colour at once (levels of at most
-// 130 x 18, 66 x 34 or 34 x 66 cells), each thread owns at most one cell of
-// each colour for the whole smoothing: its cells' rules
-// are decoded once, and a colour phase is the five reads of p, the update
-// and one write.
-__device__ __forceinline__ void lds_sweeps(float *P, const float *Fv, const uint8_t *M, int w,
-                                           int h, float hh, float alpha, int nu) {
-  const RowGroups q = row_groups((w - 1) >> 1);
-  if (q.step >= h - 2 && 2 * q.L >= w - 2) {
-    const int y = 1 + q.r0;
-    const int xa = 1 + ((1 + q.r0) & 1) + 2 * q.lr; // colour 0
-    const int xb = 1 + ((2 + q.r0) & 1) + 2 * q.lr; // colour 1
-    const bool oka = y < h - 1 && xa < w - 1, okb = y < h - 1 && xb < w - 1;
-    const int ia = y * w + xa, ib = y * w + xb;
-    CellRule ra{}, rb{};
-    if (oka) ra = cell_rule(M[ia], Fv[ia], hh);
-    if (okb) rb = cell_rule(M[ib], Fv[ib], hh);
-    for (int s = 0; s < nu; s++) {
-      if (oka) P[ia] = smooth_rule(P[ia], P[ia - 1], P[ia + 1], P[ia - w], P[ia + w], ra, alpha);
-      __syncthreads();
-      if (okb) P[ib] = smooth_rule(P[ib], P[ib - 1], P[ib + 1], P[ib - w], P[ib + w], rb, alpha);
-      __syncthreads();
-    }
-    return;
-  }
-  for (int s = 0; s < nu; s++)
-    for (int color = 0; color < 2; color++) {
-      const int x0 = 1 + ((1 + q.r0 + color) & 1) + 2 * q.lr;
-      for (int y = 1 + q.r0; y < h - 1; y += q.step) {
-        for (int x = x0; x < w - 1; x += 2 * q.L) {
-          int i = y * w + x;
-          P[i] = smooth(P[i], P[i - 1], P[i + 1], P[i - w], P[i + w], Fv[i], M[i], hh, alpha);
-        }
-      }
-      __syncthreads();
-    }
+// residual_of with the rule's selectors (f itself beside the rule)
+__device__ __forceinline__ float residual_rule(float pc, float po, float pp, float ps, float pn,
+                                               float fv, const CellRule &c, float ihsq) {
+  float val = 0.0f;
+  val += pick(c.so, po, pc);
+  val += pick(c.sp, pp, pc);
+  val += pick(c.ss, ps, pc);
+  val += pick(c.sn, pn, pc);
+  val += -4.0f * pc;
+  val *= ihsq;
+  return c.F != 0.0f ? fv + val : 0.0f;
 }
 
-__device__ __forceinline__ float lds_residual(const float *P, const float *Fv, const uint8_t *M,
-                                              int i, int w, float ihsq) {
-  return residual_of(P[i], P[i - 1], P[i + 1], P[i - w], P[i + w], Fv[i], M[i], ihsq);
+// flag count + the double literal 0.0001, stored as float (pressure_solver.cpp:149)
+__device__ __forceinline__ float eps_sum(int s) { return (float)((double)s + 0.0001); }
+
+// one level in LDS; planes: red at [0], black at [half]
+struct LdsLevel {
+  float *P, *Fv;
+  uint8_t *M;
+  int w, h, n, half; // cells, entries of a plane (= pairs)
+  float hh, ihsq, iw;
+  // row of cell i: (i + 1/2) / w is at least 1 / (2 w) from an integer, more
+  // than the product's rounding error for any i in LDS
+  __device__ __forceinline__ int row_of(int i) const { return (int)(((float)i + 0.5f) * iw); }
+  __device__ __forceinline__ float *plane(float *base, int black) const {
+    return base + (black ? half : 0);
+  }
+};
+__device__ __forceinline__ LdsLevel lds_level(const CoarseArgs &a, char *smem, int l) {
+  LdsLevel L;
+  L.P = (float *)(smem + a.op[l]);
+  L.Fv = (float *)(smem + a.of[l]);
+  L.M = (uint8_t *)(smem + a.om[l]);
+  L.w = a.w[l];
+  L.h = a.h[l];
+  L.n = L.w * L.h;
+  L.half = (L.n + 1) >> 1;
+  L.hh = a.hh[l];
+  L.ihsq = a.ihsq[l];
+  L.iw = a.iw[l];
+  return L;
+}
+
+// ordering of a phase's LDS writes before the next phase's reads: a level
+// whose pairs all belong to one wave needs no barrier (a wave's LDS
+// operations execute in order)
+__device__ __forceinline__ void phase_end(bool one_wave) {
+  if (one_wave) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  else __syncthreads();
+}
+
+// The thread's K pairs of a level.  r: the pair's red cell, b: its black one.
+template <int K> struct LevelPairs {
+  int t[K], i0[K];                // pair, its first cell
+  int x0[K], y0[K];               // column and row of the first cell
+  bool rfirst[K];                 // the first cell is the red one
+  bool okr[K], okb[K];            // interior
+  int ro[K], rs[K], rn[K];        // the red cell's outside, south, north entries (black plane)
+  int bo[K], bs[K], bn[K];        // the black cell's (red plane)
+  float pr[K], pb[K], fr[K], fb[K];
+  CellRule rr[K], rb[K];
+
+  __device__ __forceinline__ void locate(const LdsLevel &L) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      t[k] = (int)threadIdx.x + k * TPB_C;
+      const int i = i0[k] = 2 * t[k];
+      const int y = y0[k] = L.row_of(i), x = x0[k] = i - y * L.w;
+      // a pair that wraps into the next row is two ring cells
+      const bool row = i < L.n && y >= 1 && y <= L.h - 2;
+      const bool ok0 = row && x >= 1 && x <= L.w - 2, ok1 = row && x + 1 <= L.w - 2;
+      const bool rf = rfirst[k] = ((x + y) & 1) != 0;
+      okr[k] = rf ? ok0 : ok1;
+      okb[k] = rf ? ok1 : ok0;
+      const int ir = rf ? i : i + 1, ib = rf ? i + 1 : i;
+      ro[k] = (2 * ir - ib) >> 1;
+      rs[k] = (ir - L.w) >> 1;
+      rn[k] = (ir + L.w) >> 1;
+      bo[k] = (2 * ib - ir) >> 1;
+      bs[k] = (ib - L.w) >> 1;
+      bn[k] = (ib + L.w) >> 1;
+    }
+  }
+  // f and the rules of the interior cells, with the pair's two masks
+  __device__ __forceinline__ void decode(const LdsLevel &L, int k, unsigned m0, unsigned m1) {
+    const unsigned mr = rfirst[k] ? m0 : m1, mb = rfirst[k] ? m1 : m0;
+    rr[k] = cell_rule(mr, rfirst[k], fr[k], L.hh);
+    rb[k] = cell_rule(mb, !rfirst[k], fb[k], L.hh);
+    // the first cell's outside neighbour lies west of the pair, the second's east
+  }
+  // f and the masks from LDS; ZERO: p is zero, else read
+  template <bool ZERO> __device__ __forceinline__ void load(const LdsLevel &L) {
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const bool any = okr[k] || okb[k];
+      fr[k] = any ? L.Fv[t[k]] : 0.0f;
+      fb[k] = any ? L.Fv[L.half + t[k]] : 0.0f;
+      const unsigned m = any ? *(const uint16_t *)(L.M + i0[k]) : 0u;
+      pr[k] = !ZERO && any ? L.P[t[k]] : 0.0f;
+      pb[k] = !ZERO && any ? L.P[L.half + t[k]] : 0.0f;
+      decode(L, k, m & 0xffu, m >> 8);
+    }
+  }
+  __device__ __forceinline__ void red(const LdsLevel &L, float alpha) {
+    float *R = L.P, *B = L.P + L.half;
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (okr[k]) {
+        pr[k] = smooth_rule(pr[k], B[ro[k]], pb[k], B[rs[k]], B[rn[k]], rr[k], alpha);
+        R[t[k]] = pr[k];
+      }
+  }
+  __device__ __forceinline__ void black(const LdsLevel &L, float alpha) {
+    float *R = L.P, *B = L.P + L.half;
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (okb[k]) {
+        pb[k] = smooth_rule(pb[k], R[bo[k]], pr[k], R[bs[k]], R[bn[k]], rb[k], alpha);
+        B[t[k]] = pb[k];
+      }
+  }
+  __device__ __forceinline__ void sweeps(const LdsLevel &L, int nu, float alpha, bool one_wave) {
+    for (int s = 0; s < nu; s++) {
+      red(L, alpha);
+      phase_end(one_wave);
+      black(L, alpha);
+      phase_end(one_wave);
+    }
+  }
+  // the interior cells' residuals into the planes at Q
+  __device__ __forceinline__ void residual(const LdsLevel &L, float *Q) {
+    const float *R = L.P, *B = L.P + L.half;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      if (okr[k])
+        Q[t[k]] = residual_rule(pr[k], B[ro[k]], pb[k], B[rs[k]], B[rn[k]], fr[k], rr[k], L.ihsq);
+      if (okb[k])
+        Q[L.half + t[k]] =
+            residual_rule(pb[k], R[bo[k]], pr[k], R[bs[k]], R[bn[k]], fb[k], rb[k], L.ihsq);
+    }
+  }
+  // prolongate + correct (pressure_solver.cpp:134-181): a cell in an even row
+  // takes coarse row y / 2, in an odd row also the one above, and likewise
+  // the columns
+  __device__ __forceinline__ void correct(const LdsLevel &L, const LdsLevel &C) {
+    auto E = [&](int i, int x, int y) { return C.plane(C.P, !((x + y) & 1))[i >> 1]; };
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      if (!(okr[k] || okb[k])) continue;
+      // the pair holds an even column xe and an odd one xo: xo = xe + 1 or,
+      // where an odd width shifts the pairs, xe - 1; coarse columns a, a + 1
+      // under the odd one
+      const bool efirst = !(x0[k] & 1);
+      const int y = y0[k], xe = efirst ? x0[k] : x0[k] + 1, xo = efirst ? x0[k] + 1 : x0[k];
+      const bool odd_row = (y & 1) != 0;
+      const int by = y >> 1, ae = xe >> 1, ao = xo >> 1;
+      const bool up = !odd_row || y <= L.h - 3; // an odd row needs the coarse row above
+      const int by1 = odd_row && up ? by + 1 : by;
+      const int ao1 = min(ao + 1, C.w - 1);
+      const int c0 = by * C.w, c1 = by1 * C.w;
+      // coarse values under the odd column (a, a + 1) x (b, b + 1); the even
+      // column is a or a + 1
+      const float e00 = E(c0 + ao, ao, by), e10 = E(c0 + ao1, ao1, by);
+      const float e01 = E(c1 + ao, ao, by1), e11 = E(c1 + ao1, ao1, by1);
+      const int f00 = C.M[c0 + ao] & MK_SELF, f10 = C.M[c0 + ao1] & MK_SELF;
+      const int f01 = C.M[c1 + ao] & MK_SELF, f11 = C.M[c1 + ao1] & MK_SELF;
+      const float g0 = ae == ao ? e00 : e10, g1 = ae == ao ? e01 : e11;
+      const int q0 = ae == ao ? f00 : f10, q1 = ae == ao ? f01 : f11;
+      const bool even_red = efirst == rfirst[k];
+      const float Fe = even_red ? rr[k].F : rb[k].F, Fo = even_red ? rb[k].F : rr[k].F;
+      const float ee = odd_row ? Fe * (g0 + g1) / eps_sum(q0 + q1) : g0 * Fe;
+      const float num = odd_row ? e00 + e11 + e10 + e01 : e00 + e10;
+      const float eo = Fo * num / eps_sum(odd_row ? f00 + f11 + f10 + f01 : f00 + f10);
+      const float de = up ? ee : 0.0f, dn = up && xo <= L.w - 3 ? eo : 0.0f;
+      if (okr[k]) L.P[t[k]] = pr[k] += even_red ? de : dn;
+      if (okb[k]) L.P[L.half + t[k]] = pb[k] += even_red ? dn : de;
+    }
+  }
+};
+
+// restrict (pressure_solver.cpp:118-132) the residual planes Q of level L
+// into the coarse level's f, a coarse cell per thread
+__device__ __forceinline__ void lds_restrict(const LdsLevel &L, const LdsLevel &C, const float *Q) {
+  const float *R = Q, *B = Q + L.half;
+  for (int i = threadIdx.x; i < C.n; i += TPB_C) {
+    const int Y = C.row_of(i), X = i - Y * C.w;
+    if (Y < 1 || Y > C.h - 2 || X < 1 || X > C.w - 2) continue;
+    const int j = (2 * Y) * L.w + 2 * X, js = j - L.w, jn = j + L.w;
+    float v = 0.0f;
+    v = B[(js - 1) >> 1] * 1.0f + R[js >> 1] * 2.0f + B[(js + 1) >> 1] * 1.0f;
+    v += R[(j - 1) >> 1] * 2.0f + B[j >> 1] * 4.0f + R[(j + 1) >> 1] * 2.0f;
+    v += B[(jn - 1) >> 1] * 1.0f + R[jn >> 1] * 2.0f + B[(jn + 1) >> 1] * 1.0f;
+    C.plane(C.Fv, !((X + Y) & 1))[i >> 1] = v * (1.0f / 16.0f);
+  }
+}
+
+// a wave that owns no pair of the level only meets its barriers
+__device__ __forceinline__ bool idle_wave(const LdsLevel &L) {
+  return __builtin_amdgcn_readfirstlane((int)threadIdx.x & ~63) >= L.half;
+}
+
+// the levels below the first one, whose residual the planes Q hold on entry:
+// down to the coarsest and back up to the second, whose p is final on return
+__device__ __forceinline__ void lds_inner(const CoarseArgs &a, char *smem, float *Q) {
+  for (int l = 1; l < a.n; l++) {
+    const LdsLevel L = lds_level(a, smem, l);
+    lds_restrict(lds_level(a, smem, l - 1), L, Q);
+    __syncthreads();
+    const bool last = l == a.n - 1;
+    const int nu = last ? a.nu_coarse : a.nu_pre;
+    const bool one_wave = L.half <= 64;
+    if (idle_wave(L)) {
+      if (!one_wave)
+        for (int s = 0; s < 2 * nu; s++) __syncthreads();
+    } else {
+      LevelPairs<1> t;
+      t.locate(L);
+      t.template load<true>(L);
+      t.sweeps(L, nu, a.alpha, one_wave);
+      if (!last) t.residual(L, Q);
+    }
+    __syncthreads();
+  }
+  for (int l = a.n - 2; l >= 1; l--) {
+    const LdsLevel L = lds_level(a, smem, l), C = lds_level(a, smem, l + 1);
+    const bool one_wave = L.half <= 64;
+    if (idle_wave(L)) {
+      if (!one_wave)
+        for (int s = 0; s < 2 * a.nu_post + 1; s++) __syncthreads();
+    } else {
+      LevelPairs<1> t;
+      t.locate(L);
+      t.template load<false>(L);
+      t.correct(L, C);
+      phase_end(one_wave);
+      t.sweeps(L, a.nu_post, a.alpha, one_wave);
+    }
+    __syncthreads();
+  }
+}
+
+// p = 0 on every level and the masks of the levels below the first one in LDS.
+// The masks' first TPB_C bytes of up to KR levels are loaded by load() in one
+// round, which the caller issues along with its own loads.
+struct CoarseInit {
+  static constexpr int KR = 4;
+  uint8_t rm[KR];
+  __device__ __forceinline__ void load(const CoarseArgs &a) {
+#pragma unroll
+    for (int r = 0; r < KR; r++)
+      if (1 + r < a.n && (int)threadIdx.x < a.w[1 + r] * a.h[1 + r])
+        rm[r] = a.mask[1 + r][threadIdx.x];
+  }
+  __device__ __forceinline__ void store(const CoarseArgs &a, char *smem) const {
+    const int tid = threadIdx.x;
+    for (int l = 0; l < a.n; l++) {
+      float *P = (float *)(smem + a.op[l]);
+      const int m = (a.w[l] * a.h[l] + 1) & ~1;
+      for (int i = tid; i < m; i += TPB_C) P[i] = 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < KR; r++)
+      if (1 + r < a.n && tid < a.w[1 + r] * a.h[1 + r])
+        ((uint8_t *)(smem + a.om[1 + r]))[tid] = rm[r];
+    for (int l = 1; l < a.n; l++) {
+      const int n = a.w[l] * a.h[l];
+      for (int i = tid + (l <= KR ? TPB_C : 0); i < n; i += TPB_C)
+        ((uint8_t *)(smem + a.om[l]))[i] = a.mask[l][i];
+    }
+  }
+};
+
+// the first level with K pairs per thread, in registers throughout.  ALONE: it
+// is the coarsest one too
+template <int K, bool ALONE>
+__device__ __forceinline__ void lds_top(const CoarseArgs &a, char *smem, const float *f0,
+                                        float *p0) {
+  const LdsLevel L = lds_level(a, smem, 0);
+  float *Q = (float *)(smem + a.orr);
+  // every load before the first wait; a second cell past the level's end is
+  // not there
+  const uint8_t *m0 = a.mask[0];
+  float fa[K], fb[K];
+  unsigned ma[K], mb[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int i = 2 * ((int)threadIdx.x + k * TPB_C);
+    const bool in0 = i < L.n, in1 = i + 1 < L.n;
+    fa[k] = in0 ? f0[i] : 0.0f;
+    fb[k] = in1 ? f0[i + 1] : 0.0f;
+    ma[k] = in0 ? m0[i] : 0u;
+    mb[k] = in1 ? m0[i + 1] : 0u;
+  }
+  CoarseInit init;
+  init.load(a);
+  LevelPairs<K> t;
+  t.locate(L);
+  init.store(a, smem);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    t.fr[k] = t.rfirst[k] ? fa[k] : fb[k];
+    t.fb[k] = t.rfirst[k] ? fb[k] : fa[k];
+    t.pr[k] = t.pb[k] = 0.0f;
+    t.decode(L, k, ma[k], mb[k]);
+  }
+  __syncthreads();
+  if (ALONE || a.n == 1) {
+    t.sweeps(L, a.nu_coarse, a.alpha, false);
+  } else {
+    t.sweeps(L, a.nu_pre, a.alpha, false);
+    t.residual(L, Q);
+    __syncthreads();
+    lds_inner(a, smem, Q);
+    t.correct(L, lds_level(a, smem, 1));
+    __syncthreads();
+    t.sweeps(L, a.nu_post, a.alpha, false);
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const float pa = t.rfirst[k] ? t.pr[k] : t.pb[k], pb = t.rfirst[k] ? t.pb[k] : t.pr[k];
+    if (t.i0[k] < L.n) p0[t.i0[k]] = pa;
+    if (t.i0[k] + 1 < L.n) p0[t.i0[k] + 1] = pb;
+  }
 }
 
 // The whole V-cycle of levels first..L-2 of one domain in LDS, by one
 // 1024-thread workgroup; f0 is the first level's rhs, the first level's
-// solution is written to p0.
+// solution is written to p0.  A first level of more than kCoarseMaxCells
+// cells is taken only where no smaller one exists (very elongated domains),
+// so it is the coarsest level too: BIG, a variant of its own because it needs
+// more registers.
+template <bool BIG>
 __device__ __forceinline__ void coarse_vcycle_body(const CoarseArgs &a, const float *f0,
                                                   float *p0) {
   extern __shared__ __align__(16) char smem[];
-  const int tid = threadIdx.x;
-  // load: f of the first level, masks of all levels; p = 0 everywhere.
-  // Each round issues KC loads per thread before its LDS stores, so a round
-  // costs one memory latency instead of one per element; the first
-  // TPB_C-element round of levels 1..KR rides in level 0's first round, so
-  // the small levels' masks cost no latency of their own.
-  constexpr int KC = 8, KR = 4;
-  // elements [from, n) of level l, KC per thread per round
-  auto stage = [&](int l, int from) {
-    float *P = (float *)(smem + a.op[l]);
-    float *Fv = (float *)(smem + a.of[l]);
-    uint8_t *M = (uint8_t *)(smem + a.om[l]);
-    const uint8_t *mg = a.mask[l];
-    const int n = a.w[l] * a.h[l];
-    for (int base = from; base < n; base += KC * TPB_C) {
-      float vf[KC];
-      uint8_t vm[KC];
-#pragma unroll
-      for (int k = 0; k < KC; k++) {
-        const int i = base + tid + k * TPB_C;
-        if (i < n) {
-          vf[k] = (l == 0) ? f0[i] : 0.0f;
-          vm[k] = mg[i];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < KC; k++) {
-        const int i = base + tid + k * TPB_C;
-        if (i < n) {
-          P[i] = 0.0f;
-          Fv[i] = vf[k];
-          M[i] = vm[k];
-        }
-      }
-    }
-  };
-  {
-    uint8_t rm[KR];
-#pragma unroll
-    for (int r = 0; r < KR; r++)
-      if (1 + r < a.n && tid < a.w[1 + r] * a.h[1 + r]) rm[r] = a.mask[1 + r][tid];
-    stage(0, 0);
-#pragma unroll
-    for (int r = 0; r < KR; r++)
-      if (1 + r < a.n && tid < a.w[1 + r] * a.h[1 + r]) {
-        const int l = 1 + r;
-        ((float *)(smem + a.op[l]))[tid] = 0.0f;
-        ((float *)(smem + a.of[l]))[tid] = 0.0f;
-        ((uint8_t *)(smem + a.om[l]))[tid] = rm[r];
-      }
-  }
-  for (int l = 1; l < a.n; l++) stage(l, l <= KR ? TPB_C : 0);
-  __syncthreads();
-
-  // descend
-  for (int l = 0; l < a.n - 1; l++) {
-    float *P = (float *)(smem + a.op[l]);
-    float *Fv = (float *)(smem + a.of[l]);
-    const uint8_t *M = (const uint8_t *)(smem + a.om[l]);
-    const int w = a.w[l], h = a.h[l];
-    lds_sweeps(P, Fv, M, w, h, a.hh[l], a.alpha, a.nu_pre);
-    // residual (pressure_solver.cpp:91-116) of every interior cell once,
-    // then restrict (:118-132) into level l+1, whose p starts at 0
-    float *Rr = (float *)(smem + a.orr);
-    float *Fc = (float *)(smem + a.of[l + 1]);
-    float *Pc = (float *)(smem + a.op[l + 1]);
-    const int wc = a.w[l + 1], hc = a.h[l + 1];
-    const float ihsq = 1.0f / a.hh[l] / a.hh[l];
-    const RowGroups qr = row_groups(w - 2);
-    for (int y = 1 + qr.r0; y < h - 1; y += qr.step)
-      for (int x = 1 + qr.lr; x < w - 1; x += qr.L)
-        Rr[y * w + x] = lds_residual(P, Fv, M, y * w + x, w, ihsq);
-    __syncthreads();
-    const RowGroups qc = row_groups(wc - 2);
-    for (int y = 1 + qc.r0; y < hc - 1; y += qc.step)
-    for (int x = 1 + qc.lr; x < wc - 1; x += qc.L) {
-      int c = (2 * y) * w + 2 * x;
-      auto R = [&](int dx, int dy) { return Rr[c + dy * w + dx]; };
-      float v = 0.0f;
-      v = R(-1, -1) * 1.0f + R(0, -1) * 2.0f + R(1, -1) * 1.0f;
-      v += R(-1, 0) * 2.0f + R(0, 0) * 4.0f + R(1, 0) * 2.0f;
-      v += R(-1, 1) * 1.0f + R(0, 1) * 2.0f + R(1, 1) * 1.0f;
-      Fc[y * wc + x] = v * (1.0f / 16.0f);
-      Pc[y * wc + x] = 0.0f;
-    }
-    __syncthreads();
-  }
-  // coarsest solved level
-  {
-    int l = a.n - 1;
-    float *P = (float *)(smem + a.op[l]);
-    float *Fv = (float *)(smem + a.of[l]);
-    const uint8_t *M = (const uint8_t *)(smem + a.om[l]);
-    lds_sweeps(P, Fv, M, a.w[l], a.h[l], a.hh[l], a.alpha, a.nu_coarse);
-  }
-  // ascend
-  for (int l = a.n - 2; l >= 0; l--) {
-    float *P = (float *)(smem + a.op[l]);
-    float *Fv = (float *)(smem + a.of[l]);
-    const uint8_t *M = (const uint8_t *)(smem + a.om[l]);
-    const int w = a.w[l], h = a.h[l];
-    const float *Pc = (const float *)(smem + a.op[l + 1]);
-    const uint8_t *Mc = (const uint8_t *)(smem + a.om[l + 1]);
-    const int wc = a.w[l + 1];
-    // prolongate + correct (pressure_solver.cpp:134-181) by 2x2 blocks of
-    // fine cells over coarse cell (ax, by), each by its parity rule
-    auto E = [&](int xx, int yy) { return Pc[yy * wc + xx]; };
-    auto FC = [&](int xx, int yy) { return (int)(Mc[yy * wc + xx] & MK_SELF); };
-    const RowGroups qp = row_groups(((w - 2) >> 1) + 1);
-    for (int by = qp.r0; by <= (h - 2) >> 1; by += qp.step)
-    for (int ax = qp.lr; ax <= (w - 2) >> 1; ax += qp.L) {
-      const float e00 = E(ax, by);
-      const int f00 = FC(ax, by);
-#pragma unroll
-      for (int dy = 0; dy < 2; dy++)
-#pragma unroll
-        for (int dx = 0; dx < 2; dx++) {
-          const int x = 2 * ax + dx, y = 2 * by + dy;
-          if (x < 1 || x > w - 2 || y < 1 || y > h - 2) continue;
-          const int i = y * w + x;
-          const float F = (M[i] & MK_SELF) ? 1.0f : 0.0f;
-          float e = 0.0f;
-          if (dx == 0 && dy == 0) {
-            e = e00 * F;
-          } else if (dy == 0) {
-            if (x <= w - 3) e = F * (e00 + E(ax + 1, by)) / eps_count(f00 + FC(ax + 1, by));
-          } else if (dx == 0) {
-            if (y <= h - 3) e = F * (e00 + E(ax, by + 1)) / eps_count(f00 + FC(ax, by + 1));
-          } else {
-            if (x <= w - 3 && y <= h - 3)
-              e = F * (e00 + E(ax + 1, by + 1) + E(ax + 1, by) + E(ax, by + 1)) /
-                  eps_count(f00 + FC(ax + 1, by + 1) + FC(ax + 1, by) + FC(ax, by + 1));
-          }
-          P[i] += e;
-        }
-    }
-    __syncthreads();
-    lds_sweeps(P, Fv, M, w, h, a.hh[l], a.alpha, a.nu_post);
-  }
-  // write the first level's solution
-  {
-    const float *P = (const float *)(smem + a.op[0]);
-    int n = a.w[0] * a.h[0];
-    for (int i = tid; i < n; i += TPB_C) p0[i] = P[i];
-  }
+  const int pairs = (a.w[0] * a.h[0] + 1) >> 1;
+  if (pairs <= TPB_C) lds_top<1, false>(a, smem, f0, p0);
+  else if (pairs <= 2 * TPB_C) lds_top<2, false>(a, smem, f0, p0);
+  else if (BIG && pairs <= 4 * TPB_C) lds_top<4, true>(a, smem, f0, p0);
+  else if (BIG) lds_top<6, true>(a, smem, f0, p0);
 }
+static_assert(kCoarseMaxCells == 4 * TPB_C && (size_t)2 * 6 * TPB_C * 13 >= LDS_BUDGET,
+              "two pairs per thread; with BIG six, at 13 bytes of LDS a cell");
+inline bool coarse_big(int w, int h) { return (size_t)w * h > kCoarseMaxCells; }
 
 // LDS layout (p, f, mask per level, 16-byte aligned) of levels first..L-2
 // for level sizes ws/hs; fills the offsets of `a` if given.  Returns the
@@ -302,6 +454,7 @@ inline size_t coarse_lds_layout(const int *ws, const int *hs, int first, int lev
     if (k >= MAXL) return (size_t)-1;
     size_t n = (size_t)ws[l] * hs[l];
     if (a) {
+      a->iw[k] = 1.0f / (float)ws[l];
       a->op[k] = (int)off;
       a->of[k] = (int)(off + ((n * 4 + 15) & ~size_t(15)));
       a->om[k] = (int)(off + 2 * ((n * 4 + 15) & ~size_t(15)));

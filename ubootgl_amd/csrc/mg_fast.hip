@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(TPB_T)
 // ---------------------------------------------------------------------------
 // single-workgroup V-cycle in LDS
 __global__ void __launch_bounds__(TPB_C) k_coarse_vcycle(CoarseArgs a) {
-  coarse_vcycle_body(a, a.f0, a.p0);
+  coarse_vcycle_body<false>(a, a.f0, a.p0);
 }
 
 } // namespace
@@ -75,7 +75,6 @@ bool coarse_fits_lds(const Level *lv, int first, int levels) {
 
 void launch_coarse_vcycle(const Level *lv, int first, int levels, float h, int nu_pre,
                           int nu_post, int nu_coarse, float alpha, hipStream_t s) {
-  static bool attr_set = false;
   CoarseArgs a{};
   size_t bytes = coarse_lds_bytes(lv, first, levels, &a);
   a.n = levels - 1 - first;
@@ -86,6 +85,7 @@ void launch_coarse_vcycle(const Level *lv, int first, int levels, float h, int n
     a.h[k] = L.h;
     a.mask[k] = L.mask;
     a.hh[k] = hl;
+    a.ihsq[k] = 1.0f / hl / hl;
     if (k + 1 < a.n) hl = hl * (L.w - 1.0f) / (lv[first + k + 1].w - 1.0f); // pressure_solver.cpp:229
   }
   a.f0 = lv[first].f;
@@ -94,11 +94,12 @@ void launch_coarse_vcycle(const Level *lv, int first, int levels, float h, int n
   a.nu_post = nu_post;
   a.nu_coarse = nu_coarse;
   a.alpha = alpha;
-  if (!attr_set) {
+  static const bool attr_set = [] { // more than 64 KiB of LDS
     (void)hipFuncSetAttribute((const void *)k_coarse_vcycle,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BUDGET);
-    attr_set = true;
-  }
+    return true;
+  }();
+  (void)attr_set;
   hipLaunchKernelGGL(k_coarse_vcycle, dim3(1), dim3(TPB_C), bytes, s, a);
 }
 
