@@ -13,9 +13,8 @@
 // row of the stage, so domains with different level counts and ping-pong
 // parities run in the same launch.  Domains whose solve has ended are
 // skipped on the device; no host round trip is needed per stage.
-#include "batch_engine.hpp"
-#include "stream_device.hpp"
-#include "tile_device.hpp"
+#include "batch_stage.hpp"
+#include "mg_device.hpp"
 
 #include <algorithm>
 #include <array>
@@ -31,69 +30,6 @@ namespace ubg {
 namespace {
 
 constexpr int TPB = 256;
-
-struct StageArgs {
-  const BLev *lev;
-  const BDom *dom;
-  const int *off; // tile prefix over domain slots [ndom + 1], tiles per row [ndom], tile width [ndom]
-  int ndom;
-  int ntiles;
-  int level;
-  const uint8_t *ia; // per-domain index row a
-  const uint8_t *ib; // per-domain index row b
-  float alpha;
-  int oty; // tile rows of the fused level passes (their widths are per domain)
-  int zg;  // row-streamed level-0 passes apply setZeroGradientBC (projection solves)
-};
-
-__device__ __forceinline__ bool dom_active(const BDom &D) {
-  return __builtin_amdgcn_readfirstlane(D.st->active) != 0;
-}
-
-// Tiles of a stage are split into equal contiguous chunks, one per block of
-// the (persistent) grid, in XCD-grouped block order so that neighbouring
-// chunks share an XCD's L2.  A block locates the domain slot of its first tile
-// once (the last d with off[d] <= t; domains without tiles at this level
-// have off[d] == off[d+1]) and then walks forward.
-struct TileWalk {
-  int t, t1; // current tile, end of the chunk
-  int d, j;  // domain slot, tile index within the domain
-  int nt, ntx, otx;
-  __device__ __forceinline__ bool init(const StageArgs &a) {
-    const int per = (a.ntiles + gridDim.x - 1) / gridDim.x;
-    const int b = xcd_tile(blockIdx.x, gridDim.x);
-    t = b * per;
-    t1 = min(t + per, a.ntiles);
-    if (t >= t1) return false;
-    int lo = 0, hi = a.ndom;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (a.off[mid] <= t) lo = mid;
-      else hi = mid;
-    }
-    d = lo;
-    j = t - a.off[d];
-    nt = a.off[d + 1] - a.off[d];
-    ntx = a.off[a.ndom + 1 + d];
-    otx = a.off[2 * a.ndom + 1 + d];
-    return true;
-  }
-  __device__ __forceinline__ bool next(const StageArgs &a) {
-    if (++t >= t1) return false;
-    if (++j == nt) {
-      do {
-        d++;
-      } while (a.off[d + 1] == a.off[d]);
-      j = 0;
-      nt = a.off[d + 1] - a.off[d];
-      ntx = a.off[a.ndom + 1 + d];
-      otx = a.off[2 * a.ndom + 1 + d];
-    }
-    return true;
-  }
-  __device__ __forceinline__ int tx() const { return j % ntx; }
-  __device__ __forceinline__ int ty() const { return j / ntx; }
-};
 
 // One red+black rbgs sweep of a TX x TY tile, ping-pong (read p[a], write
 // p[a^1]).  p is staged with a 2-cell halo; red cells ((x+y) odd) of the tile
@@ -263,136 +199,6 @@ __global__ void __launch_bounds__(TPB) kb_pc(StageArgs a) {
       p[i] += e;
     }
   } while (tw.next(a));
-}
-
-// The fused level passes of tile_device.hpp over the tiles of every member
-// domain at one level (each domain's own even column split, oty rows, walked
-// as the other stages): pre reads p[ia], writes p[ia^1], the coarse rhs and
-// a zero coarse p[ib]; post reads p[ia] and the coarse solution p[ib],
-// writes p[ia^1].  ZP (every level below the finest): p[ia] is the zero
-// solution the restriction above wrote, and pre does not read it.
-template <int NU, int TPB_T, bool ZP>
-__global__ void __launch_bounds__(TPB_T) kb_tile_pre(StageArgs a) {
-  extern __shared__ __align__(16) char smem[];
-  TileWalk tw;
-  if (!tw.init(a)) return;
-  do {
-    const BDom &D = a.dom[tw.d];
-    if (!dom_active(D)) continue;
-    const BLev &F = a.lev[tw.d * BMAXL + a.level];
-    const BLev &C = a.lev[tw.d * BMAXL + a.level + 1];
-    const int s = a.ia[tw.d];
-    __syncthreads(); // the previous tile's LDS readers are done
-    tile_pre_body<NU, TPB_T, ZP>(smem, tw.tx() * tw.otx, tw.ty() * a.oty, tw.otx, a.oty,
-                                 F.p[s], F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                                 F.ihsq, C.f, C.p[a.ib[tw.d]], C.w, C.h);
-  } while (tw.next(a));
-}
-template <int NU, int TPB_T>
-__global__ void __launch_bounds__(TPB_T) kb_tile_post(StageArgs a) {
-  extern __shared__ __align__(16) char smem[];
-  TileWalk tw;
-  if (!tw.init(a)) return;
-  do {
-    const BDom &D = a.dom[tw.d];
-    if (!dom_active(D)) continue;
-    const BLev &F = a.lev[tw.d * BMAXL + a.level];
-    const BLev &C = a.lev[tw.d * BMAXL + a.level + 1];
-    const int s = a.ia[tw.d];
-    __syncthreads();
-    tile_post_body<NU, TPB_T>(smem, tw.tx() * tw.otx, tw.ty() * a.oty, tw.otx, a.oty, F.p[s],
-                              F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                              C.p[a.ib[tw.d]], C.mask, C.w, C.h);
-  } while (tw.next(a));
-}
-
-// Row-streamed level passes (stream_device.hpp) over the units (strip x row
-// block, one wave each) of every member domain whose level is streamed.  A
-// wave finds its domain slot in the unit prefix (the last d with off[d] <=
-// unit, as the tile walk does); the table's second and third rows hold the
-// domain's strip count and row-block height.
-struct StreamUnit {
-  int d, unit, nstrips, R;
-};
-__device__ __forceinline__ bool stream_unit(const StageArgs &a, StreamUnit &u) {
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g = xcd_tile(blockIdx.x, gridDim.x) * (TPB / 64) + wid;
-  if (g >= a.ntiles) return false; // whole wave leaves together
-  int lo = 0, hi = a.ndom;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (a.off[mid] <= g) lo = mid;
-    else hi = mid;
-  }
-  u.d = lo;
-  u.unit = g - a.off[lo];
-  u.nstrips = a.off[a.ndom + 1 + lo];
-  u.R = a.off[2 * a.ndom + 1 + lo];
-  return true;
-}
-
-// one red+black sweep: reads p[ia], writes p[ia^1]
-__global__ void __launch_bounds__(TPB) kb_stream_sweep(StageArgs a) {
-  StreamUnit u;
-  if (!stream_unit(a, u)) return;
-  if (!dom_active(a.dom[u.d])) return;
-  const BLev &F = a.lev[u.d * BMAXL + a.level];
-  const int s = a.ia[u.d];
-  const bool al = (F.w & 1) == 0;
-  if (a.zg) {
-    if (al)
-      rbgs_pair_unit<true, true>(F.p[s], F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                                 u.nstrips, u.R, u.unit);
-    else
-      rbgs_pair_unit<true, false>(F.p[s], F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                                  u.nstrips, u.R, u.unit);
-  } else if (al) {
-    rbgs_pair_unit<false, true>(F.p[s], F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                                u.nstrips, u.R, u.unit);
-  } else {
-    rbgs_pair_unit<false, false>(F.p[s], F.p[s ^ 1], F.f, F.mask, F.w, F.h, F.hh, a.alpha,
-                                 u.nstrips, u.R, u.unit);
-  }
-}
-
-// MODE_RR: last pre-sweep + residual + restriction (coarse rhs, zero coarse
-// p[ib]); MODE_PC: prolongation of the coarse p[ib] + correction + first
-// post-sweep.  Both read p[ia] and write p[ia^1].
-template <int MODE>
-__global__ void __launch_bounds__(TPB) kb_stream_pass(StageArgs a) {
-  StreamUnit u;
-  if (!stream_unit(a, u)) return;
-  if (!dom_active(a.dom[u.d])) return;
-  const BLev &F = a.lev[u.d * BMAXL + a.level];
-  const BLev &C = a.lev[u.d * BMAXL + a.level + 1];
-  const int s = a.ia[u.d];
-  StreamArgs A{};
-  A.src = F.p[s];
-  A.dst = F.p[s ^ 1];
-  A.f = F.f;
-  A.m = F.mask;
-  A.w = F.w;
-  A.h = F.h;
-  A.hh = F.hh;
-  A.alpha = a.alpha;
-  A.ihsq = F.ihsq;
-  A.crc = C.f;
-  A.cec = C.p[a.ib[u.d]];
-  A.cpin = C.p[a.ib[u.d]];
-  A.cmask = C.mask;
-  A.wc = C.w;
-  A.hc = C.h;
-  A.nstrips = u.nstrips;
-  A.R = u.R;
-  const bool al = (F.w & 1) == 0;
-  if (a.zg) {
-    if (al) mg_stream_unit<1, MODE, true, true>(A, u.unit);
-    else mg_stream_unit<1, MODE, true, false>(A, u.unit);
-  } else if (al) {
-    mg_stream_unit<1, MODE, false, true>(A, u.unit);
-  } else {
-    mg_stream_unit<1, MODE, false, false>(A, u.unit);
-  }
 }
 
 // the coarse levels of each domain in LDS, one workgroup per domain slot;
@@ -605,30 +411,8 @@ bool shape_ok(int tx, int ty) {
 
 size_t al(size_t n) { return align_up(n, 256); }
 
-// rows of the fused-pass tiles the tuning may fix (0: chosen per level)
+// tile shapes of the level passes the tuning may fix (0: chosen per level)
 bool pass_rows_ok(int r) { return r == 0 || r == 8 || r == 16 || r == 32; }
-
-void launch_tile_pass(bool pre, int nu, int tpb, int blocks, hipStream_t s, const StageArgs &a) {
-  const size_t shm = pre ? tile_pre_lds(a.oty, nu) : tile_post_lds(a.oty, nu);
-#define UBG_TP(N, T)                                                                            \
-  if (nu == N && tpb == T) {                                                                    \
-    if (pre && a.level > 0)                                                                     \
-      hipLaunchKernelGGL((kb_tile_pre<N, T, true>), dim3(blocks), dim3(T), shm, s, a);         \
-    else if (pre)                                                                               \
-      hipLaunchKernelGGL((kb_tile_pre<N, T, false>), dim3(blocks), dim3(T), shm, s, a);        \
-    else hipLaunchKernelGGL((kb_tile_post<N, T>), dim3(blocks), dim3(T), shm, s, a);           \
-    return;                                                                                     \
-  }
-  UBG_TP(0, 512)
-  UBG_TP(1, 512)
-  UBG_TP(2, 512)
-  UBG_TP(3, 512)
-  UBG_TP(0, 1024)
-  UBG_TP(1, 1024)
-  UBG_TP(2, 1024)
-  UBG_TP(3, 1024)
-#undef UBG_TP
-}
 
 } // namespace
 
@@ -1066,28 +850,6 @@ int BatchEngine::build_tables() {
 // Per stage kind and level: the prefix of tile counts over the member slots
 // and each domain's tiles per row; kernels locate their tile from these, so
 // a member change rebuilds O(domains x levels) integers, not tile lists.
-// Row-streamed levels: at least kStreamMinW wide and kStreamMinCells large,
-// with both smoothing counts >= 1 (the grid-transfer passes carry one sweep
-// each) and at most 3 (the tiled mode); row blocks of kStreamR rows; used at
-// a level only when the members' sweep units there reach kStreamMinUnits.
-// Measured on gfx950 (256 uneven batched domains and the served mix): below
-// about 4096 units a level is faster as LDS tiles; above, streaming its
-// >= 512-wide, >= 2^18-cell domains gained ~3% on the served mix and was
-// neutral on the batch.
-constexpr int kStreamMinW = 512;
-constexpr size_t kStreamMinCells = size_t(1) << 18;
-constexpr long kStreamMinUnits = 4096;
-constexpr int kStreamR = 16;
-static_assert(kStreamR % 2 == 0, "streamed passes need an even row-block height");
-
-bool BatchEngine::stream_eligible(const BGeom &G, int l) const {
-  if (l < G.cfirst && tiled() && prm_.nu_pre >= 1 && prm_.nu_post >= 1 && l == 0 &&
-      force_stream0_)
-    return true;
-  return l < G.cfirst && tiled() && prm_.nu_pre >= 1 && prm_.nu_post >= 1 &&
-         G.w[l] >= kStreamMinW && (size_t)G.w[l] * G.h[l] >= kStreamMinCells;
-}
-
 int BatchEngine::build_tiles() {
   h_off_.clear();
   // per span: tile prefix over the domain slots [nd + 1], tiles per row [nd]
@@ -1113,14 +875,6 @@ int BatchEngine::build_tiles() {
   const int tx = tune_.tx, ty = tune_.ty;
   const int nr = (int)run_.size();
   for (int l = 0; l < BMAXL; l++) {
-    long units = 0;
-    for (int s = 0; s < nr; s++) {
-      const BGeom &G = *run_[s]->g;
-      if (stream_eligible(G, l)) units += (long)cdiv(G.w[l], SW2) * cdiv(G.h[l] - 2, kStreamR);
-    }
-    stream_on_[l] = units >= kStreamMinUnits || (l == 0 && force_stream0_);
-  }
-  for (int l = 0; l < BMAXL; l++) {
     span(sw_[l], nr, [&](int s, int &nx, int &ny, int &) {
       const BGeom &G = *run_[s]->g;
       if (l >= G.cfirst) return;
@@ -1140,66 +894,36 @@ int BatchEngine::build_tiles() {
       ny = cdiv(G.h[l] - 2, PCH);
     });
   }
-  // Fused passes: each domain's columns split evenly (tile_cols); the rows
-  // fixed by the tuning, or per level the fewest (even, 8 to 32) whose tiles
-  // over all member domains fit in one residency wave of the launch's
-  // target, with 512-thread workgroups for levels of at least kTileBigCells
-  // cells in total and 1024-thread ones below.
-  auto fused = [&](Span *out, int nu) {
-    for (int l = 0; l < BMAXL; l++) {
-      size_t cells = 0;
+  // Level passes: one tile shape per level, by the tuning or by the number of
+  // 128 x 32 regions of its members (the single-domain rule over all of
+  // them); each domain's columns split evenly.
+  auto passes = [&](Span *out, bool pre, int nu) {
+    for (int l = 0; l < BMAXL && tiled(); l++) {
+      int ox0 = 0, oy0 = 0;
+      pass_tile(PASS_SMALL, true, nu, &ox0, &oy0);
+      long tiles = 0;
       for (int s = 0; s < nr; s++) {
         const BGeom &G = *run_[s]->g;
-        if (l < G.cfirst && !streamed(G, l)) cells += (size_t)G.w[l] * G.h[l];
+        if (l < G.cfirst) tiles += (long)cdiv(G.w[l], ox0) * cdiv(G.h[l], oy0);
       }
-      const int tpb = cells >= kTileBigCells ? 512 : 1024;
-      int oty = tune_.prow;
-      if (oty == 0) {
-        auto tiles = [&](int r) {
-          long t = 0;
-          for (int s = 0; s < nr; s++) {
-            const BGeom &G = *run_[s]->g;
-            if (l >= G.cfirst || streamed(G, l)) continue;
-            int ox, nx;
-            tile_cols(G.w[l], nu, ox, nx);
-            t += (long)nx * cdiv(G.h[l], r);
-          }
-          return t;
-        };
-        oty = 8;
-        while (oty < 32 && tiles(oty) > tile_target(tpb)) oty += 2;
-      }
+      PassShape shape = tiles <= 256 ? PASS_SMALL : (tiles <= 1024 ? PASS_MID : PASS_BIG);
+      if (tune_.prow) shape = tune_.prow == 8 ? PASS_SMALL : (tune_.prow == 16 ? PASS_MID : PASS_BIG);
+      int otx = 0, oty = 0;
+      pass_tile(shape, pre, nu, &otx, &oty);
       out[l].oty = oty;
-      out[l].tpb = tpb;
+      out[l].shape = shape;
       span(out[l], nr, [&](int s, int &nx, int &ny, int &ox) {
         const BGeom &G = *run_[s]->g;
-        if (l >= G.cfirst || streamed(G, l)) return;
-        tile_cols(G.w[l], nu, ox, nx);
+        if (l >= G.cfirst) return;
+        nx = cdiv(G.w[l], otx);
+        ox = (cdiv(G.w[l], nx) + 1) & ~1;
+        nx = cdiv(G.w[l], ox);
         ny = cdiv(G.h[l], oty);
       });
     }
   };
-  fused(tp_, prm_.nu_pre);
-  fused(tq_, prm_.nu_post);
-  // row-streamed levels: units = strips x row blocks (the table's third row
-  // holds the row-block height)
-  constexpr int own_pass = 2 * (64 - 2 * (1 + 2)); // columns per strip, one-sweep passes
-  for (int l = 0; l < BMAXL; l++) {
-    span(ss_[l], nr, [&](int s, int &nx, int &ny, int &r) {
-      const BGeom &G = *run_[s]->g;
-      if (!streamed(G, l)) return;
-      nx = cdiv(G.w[l], SW2);
-      ny = cdiv(G.h[l] - 2, kStreamR);
-      r = kStreamR;
-    });
-    span(st_[l], nr, [&](int s, int &nx, int &ny, int &r) {
-      const BGeom &G = *run_[s]->g;
-      if (!streamed(G, l)) return;
-      nx = cdiv(G.w[l], own_pass);
-      ny = cdiv(G.h[l], kStreamR);
-      r = kStreamR;
-    });
-  }
+  passes(tp_, true, prm_.nu_pre);
+  passes(tq_, false, prm_.nu_post);
   span(upd_, (int)all_.size(), [&](int s, int &nx, int &ny, int &) {
     nx = all_[s]->gx;
     ny = all_[s]->gy;
@@ -1216,7 +940,7 @@ int BatchEngine::build_tiles() {
   return UBG_OK;
 }
 
-enum { ST_SWEEP, ST_RR, ST_PC, ST_COARSE, ST_UPDATE, ST_NORM, ST_TPRE, ST_TPOST, ST_SSWEEP, ST_SRR, ST_SPC };
+enum { ST_SWEEP, ST_RR, ST_PC, ST_COARSE, ST_UPDATE, ST_NORM, ST_TPRE, ST_TPOST };
 
 // One V-cycle of the running members in the tiled mode (the per-level
 // passes of solveLevel, pressure_solver.cpp:201-248), simulated on (and
@@ -1230,50 +954,25 @@ void BatchEngine::gen_vcycle_tiled(std::vector<StageRec> &st, std::vector<uint8_
     st.push_back(StageRec{kind, level, off});
     return {idx.data() + off, idx.data() + off + n};
   };
-  // per level: a streamed domain takes nu_pre - 1 sweeps and the fused
-  // pre pass (each flipping the level's p), a tiled one the fused tile
-  // pre pass (one flip); mirrored on the way up
-  auto tile_at = [&](size_t d, int l) {
-    return l < run_[d]->g->cfirst && !streamed(*run_[d]->g, l);
-  };
-  auto stream_at = [&](size_t d, int l) { return streamed(*run_[d]->g, l); };
-  auto sweep_rows = [&](int l, int n) {
-    for (int k = 0; k < n; k++) {
-      auto r = row(ST_SSWEEP, l);
-      for (size_t d = 0; d < nr; d++)
-        if (stream_at(d, l)) {
-          r.first[d] = (uint8_t)run_[d]->cur[l];
-          run_[d]->cur[l] ^= 1;
-        }
-    }
-  };
-  auto pass_row = [&](int kind, int l, auto at) {
+  // per level one pass on the way down and one on the way up, each flipping
+  // the level's p
+  auto pass_row = [&](int kind, int l) {
     auto r = row(kind, l);
     for (size_t d = 0; d < nr; d++)
-      if (at(d, l)) {
+      if (l < run_[d]->g->cfirst) {
         r.first[d] = (uint8_t)run_[d]->cur[l];
         r.second[d] = (uint8_t)run_[d]->cur[l + 1];
         run_[d]->cur[l] ^= 1;
       }
   };
-  for (int l = 0; l < lmax_; l++) {
-    if (st_[l].n) {
-      sweep_rows(l, prm_.nu_pre - 1);
-      pass_row(ST_SRR, l, stream_at);
-    }
-    if (tp_[l].n) pass_row(ST_TPRE, l, tile_at);
-  }
+  for (int l = 0; l < lmax_; l++)
+    if (tp_[l].n) pass_row(ST_TPRE, l);
   {
     auto r = row(ST_COARSE, 0);
     for (size_t d = 0; d < nr; d++) r.first[d] = (uint8_t)run_[d]->cur[run_[d]->g->cfirst];
   }
-  for (int l = lmax_ - 1; l >= 0; l--) {
-    if (st_[l].n) {
-      pass_row(ST_SPC, l, stream_at);
-      sweep_rows(l, prm_.nu_post - 1);
-    }
-    if (tq_[l].n) pass_row(ST_TPOST, l, tile_at);
-  }
+  for (int l = lmax_ - 1; l >= 0; l--)
+    if (tq_[l].n) pass_row(ST_TPOST, l);
 }
 
 // The stage sequence of nsteps refinement steps and, per stage, the two
@@ -1370,7 +1069,6 @@ int BatchEngine::launch_stages(const std::vector<StageRec> &st, const uint8_t *d
     a.lev = d_lev_;
     a.dom = d_dom_;
     a.level = r.level;
-    a.zg = zg0_ && r.level == 0;
     a.ia = d_idx + r.off;
     a.ib = d_idx + r.off + n;
     a.alpha = prm_.alpha;
@@ -1388,36 +1086,21 @@ int BatchEngine::launch_stages(const std::vector<StageRec> &st, const uint8_t *d
       if (a.ntiles) hipLaunchKernelGGL(kb_pc, dim3(grid(a.ntiles)), dim3(TPB), 0, stream_, a);
       break;
     case ST_TPRE:
-      use(a, tp_[r.level]);
-      a.oty = tp_[r.level].oty;
+    case ST_TPOST: {
+      const bool pre = r.kind == ST_TPRE;
+      const Span &sp = pre ? tp_[r.level] : tq_[r.level];
+      use(a, sp);
+      a.oty = sp.oty;
       if (a.ntiles)
-        launch_tile_pass(true, prm_.nu_pre, tp_[r.level].tpb, grid(a.ntiles), stream_, a);
+        launch_batch_pass(sp.shape, pre, pre ? prm_.nu_pre : prm_.nu_post, zg0_, grid(a.ntiles),
+                          stream_, a);
       break;
-    case ST_TPOST:
-      use(a, tq_[r.level]);
-      a.oty = tq_[r.level].oty;
-      if (a.ntiles)
-        launch_tile_pass(false, prm_.nu_post, tq_[r.level].tpb, grid(a.ntiles), stream_, a);
-      break;
-    case ST_SSWEEP:
-      use(a, ss_[r.level]);
-      if (a.ntiles)
-        hipLaunchKernelGGL(kb_stream_sweep, dim3((a.ntiles + TPB / 64 - 1) / (TPB / 64)),
-                           dim3(TPB), 0, stream_, a);
-      break;
-    case ST_SRR:
-    case ST_SPC:
-      use(a, st_[r.level]);
-      if (a.ntiles) {
-        const dim3 g((a.ntiles + TPB / 64 - 1) / (TPB / 64));
-        if (r.kind == ST_SRR) hipLaunchKernelGGL(kb_stream_pass<MODE_RR>, g, dim3(TPB), 0, stream_, a);
-        else hipLaunchKernelGGL(kb_stream_pass<MODE_PC>, g, dim3(TPB), 0, stream_, a);
-      }
-      break;
+    }
     case ST_COARSE:
       if (!run_.empty())
-        hipLaunchKernelGGL((coarse_big_ ? kb_coarse<true> : kb_coarse<false>), dim3((unsigned)run_.size()), dim3(TPB_C), coarse_lds_,
-                           stream_, a, (const CoarseArgs *)d_cargs_, (int)run_.size());
+        hipLaunchKernelGGL((coarse_big_ ? kb_coarse<true> : kb_coarse<false>),
+                           dim3((unsigned)run_.size()), dim3(TPB_C), coarse_lds_, stream_, a,
+                           (const CoarseArgs *)d_cargs_, (int)run_.size());
       break;
     case ST_UPDATE:
       use(a, upd_);
@@ -1548,20 +1231,11 @@ int BatchEngine::run_steps_graph(int nsteps) {
   return UBG_OK;
 }
 
-int BatchEngine::set_level0_streamed(bool on) {
-  if (on == force_stream0_) return UBG_OK;
-  force_stream0_ = on;
-  drop_graphs();
-  if (d_lev_) UBG_TRY(build_tiles());
-  return UBG_OK;
-}
-
 int BatchEngine::enqueue_vcycles(int ncycles, bool zg) {
   if (!tiled() || prm_.nu_pre < 1 || prm_.nu_post < 1)
     return fail(UBG_E_INVALID, "projection batches need 1..3 pre- and post-smoothing sweeps");
   if (!fresh_.empty()) return fail(UBG_E_STATE, "projection batches take running members only");
   if (run_.empty() || ncycles <= 0) return UBG_OK;
-  UBG_TRY(set_level0_streamed(zg));
   // one captured graph per index state (the V-cycles of all members, their
   // index rows in a device buffer of the graph's own), replayed
   const std::string key =
@@ -1654,7 +1328,7 @@ int BatchEngine::launch_sweeps_only(int reps) {
   return UBG_OK;
 }
 
-// the fused pre passes of every member level, then the post passes, `reps`
+// the pre passes of every member level, then the post passes, `reps`
 // times (scratch buffers only, as launch_sweeps_only)
 int BatchEngine::launch_passes_only(int reps) {
   const int n = (int)all_.size();
@@ -1676,7 +1350,8 @@ int BatchEngine::launch_passes_only(int reps) {
     a.ntiles = sp.n;
     a.oty = sp.oty;
     int b = tune_.blocks > 0 ? std::min(a.ntiles, tune_.blocks) : a.ntiles;
-    launch_tile_pass(pre, pre ? prm_.nu_pre : prm_.nu_post, sp.tpb, std::max(b, 1), stream_, a);
+    launch_batch_pass(sp.shape, pre, pre ? prm_.nu_pre : prm_.nu_post, false, std::max(b, 1),
+                      stream_, a);
   };
   for (int r = 0; r < reps; r++) {
     for (int l = 0; l < lmax_; l++) pass(true, l);
@@ -1687,7 +1362,7 @@ int BatchEngine::launch_passes_only(int reps) {
 }
 
 // Times the candidate shapes over the member levels and keeps the fastest:
-// the fused passes' tile rows x block counts when the levels run as fused
+// the level passes' tile shapes x block counts when the levels run as
 // passes, else the smoother tile shapes x block counts.
 int BatchEngine::autotune(double *best_ms) {
   const Tuning saved = tune_;
@@ -2185,7 +1860,6 @@ UBG_API int ubg_batch_solve(ubg_batch *b, const ubg_ir_params *prm, int *graph_r
   }
   b->eng.set_vcycles(P.vcycles_per_iter);
   b->proj_active = false;
-  UBG_TRY(b->eng.set_level0_streamed(false));
   for (auto *d : b->doms) UBG_TRY(b->eng.domain_start(d, P.tol, P.max_iter));
   // first update of every domain (r0), then replayed two-step graphs
   UBG_TRY(b->eng.set_members(b->doms, {}));
@@ -2285,7 +1959,6 @@ UBG_API int ubg_batch_autotune(ubg_batch *b, const char *db_path, ubg_batch_tuni
       }
     }
   }
-  UBG_TRY(b->eng.set_level0_streamed(false));
   UBG_TRY(b->eng.set_members(b->doms, {}));
   double ms = 0.0;
   UBG_TRY(b->eng.autotune(&ms));

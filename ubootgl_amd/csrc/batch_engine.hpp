@@ -99,9 +99,12 @@ struct BDomain {
   int xcur = 0;
 };
 
+// tile shapes of the level passes: 16 waves of 2 rows, 8 of 4, 8 of 6
+enum PassShape { PASS_SMALL, PASS_MID, PASS_BIG };
+
 struct Tuning {
   int tx = 64, ty = 8, blocks = 0; // smoother tile (sweep stages), workgroups per launch
-  int prow = 0;                    // rows of the fused-pass tiles (0: chosen per level)
+  int prow = 0;                    // tile shape of the level passes (0: chosen per level)
 };
 
 // Level sizes, first LDS level and byte counts of a W x H domain.
@@ -171,14 +174,8 @@ public:
   // ncycles plain FP32 V-cycles (MG::solve, pressure_solver.cpp:250-257) of
   // every running member on its level-0 pressure and rhs; zg: level 0 takes
   // setZeroGradientBC after every sweep and after the correction (the
-  // simulation's projection).  Level 0 then runs as row-streamed passes for
-  // every domain (they carry the boundary copy); needs 1 <= nu_pre, nu_post
-  // <= 3.
+  // simulation's projection); needs 1 <= nu_pre, nu_post <= kNuPass.
   int enqueue_vcycles(int ncycles, bool zg);
-  // level 0 as row-streamed passes for every member domain (projection
-  // solves) or by the size rule (refinement solves); rebuilds the tile maps
-  // when it changes
-  int set_level0_streamed(bool on);
   int active_count() const { return *count_host_; }
   // members whose solve was still active at the last completed step
   std::vector<BDomain *> active_members() const;
@@ -228,25 +225,14 @@ private:
     size_t off = 0; // into the int array
     int n = 0;      // tiles
     int nd = 0;     // domain slots covered
-    int oty = 0;    // fused passes: tile rows
-    int tpb = 512;  //   and workgroup size
+    int oty = 0;    // level passes: tile rows
+    PassShape shape = PASS_SMALL; //   and shape
   };
   Span sw_[BMAXL], rr_[BMAXL], pc_[BMAXL], upd_;
-  Span tp_[BMAXL], tq_[BMAXL]; // fused level passes (pre, post)
-  Span ss_[BMAXL], st_[BMAXL]; // row-streamed levels: sweeps, pre / post passes
-  bool stream_on_[BMAXL] = {};  // level l has enough streamed units over the members
-  bool force_stream0_ = false;  // level 0 streamed for every domain (projection solves)
+  Span tp_[BMAXL], tq_[BMAXL]; // level passes (pre, post)
   bool zg0_ = false;            // the stages being launched apply ZG at level 0
-  // levels run as fused tile passes (smoothing counts with a tiled pass)
+  // levels run as the pre / post passes (smoothing counts that they take)
   bool tiled() const { return prm_.nu_pre <= kNuPass && prm_.nu_post <= kNuPass; }
-  // level l of a domain of this shape may run as row-streamed passes (wide
-  // and large levels) ...
-  bool stream_eligible(const BGeom &G, int l) const;
-  // ... and does, when the member domains' streamed units at that level are
-  // enough to fill the GPU (else the LDS tiles cost less per cell)
-  bool streamed(const BGeom &G, int l) const {
-    return l < BMAXL && stream_on_[l] && stream_eligible(G, l);
-  }
   int launch_passes_only(int reps);
   // stage index rows
   uint8_t *d_idx_ = nullptr;

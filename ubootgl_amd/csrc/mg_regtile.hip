@@ -84,9 +84,9 @@ template <class T> struct PostLaunch {
 // 3072x1536 at 3/3: 29.2 + 27.0 us against 32.6 + 28.9 us with 4).
 template <int NU, template <class> class Launch, typename... Args>
 void launch_shape(const Level &L, Args &&...args) {
-  using Small = RegTile<NU, 2, 16>;
-  using Mid = RegTile<NU, 4, 8>;
-  using Big = RegTile<NU, 6, 8>;
+  using Small = RegTileSmall<NU>;
+  using Mid = RegTileMid<NU>;
+  using Big = RegTileBig<NU>;
   const long tiles = (long)((L.w + Small::OTXP - 1) / Small::OTXP) *
                      ((L.h + Small::OTYP - 1) / Small::OTYP);
   if (tiles <= 256) Launch<Small>::run(args...);

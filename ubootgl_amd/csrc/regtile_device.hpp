@@ -32,9 +32,47 @@
 // sweeps; other rows take the constants from the LDS rule table.
 #pragma once
 
-#include "stream_device.hpp"
+#include "mg_device.hpp"
 
 namespace ubg {
+
+// The smoothing constants of every mask byte, for passes that look them up
+// in LDS instead of decoding the byte at each update: entry 2 mk holds the
+// four neighbour selectors (0 / -1 for the bits W, E, S, N), entry 2 mk + 1
+// RN(1/s) and -s for the neighbour count s, the quotient's select (0 when
+// s == 0, else -1) and F, as bits.  Filled by the whole workgroup.
+constexpr int kRuleEntries = 512;
+__device__ __forceinline__ void fill_rule_table(uint4 *tab) {
+  for (unsigned mk = threadIdx.x; mk < 256u; mk += blockDim.x) {
+    const unsigned s = mk >> 5;
+    const float pow2 = __int_as_float((int)((127u - (s >> 1)) << 23));
+    const float inv = (s == 3u) ? (1.0f / 3.0f) : pow2;
+    tab[2 * mk] = make_uint4(0u - ((mk >> 1) & 1u), 0u - ((mk >> 2) & 1u), 0u - ((mk >> 3) & 1u),
+                             0u - ((mk >> 4) & 1u));
+    tab[2 * mk + 1] = make_uint4(__float_as_uint(inv), __float_as_uint(-(float)s),
+                                 s == 0u ? 0u : ~0u, __float_as_uint((float)(mk & MK_SELF)));
+  }
+}
+// smooth_fhh with the mask's constants from the table: the same operations
+// in the same order (keep_if, div_count, the zero-count case, F), so the
+// same value.
+__device__ __forceinline__ float smooth_tab(float pc, float pw, float pe, float ps, float pn,
+                                            float fhh, const uint4 *tab, unsigned mk,
+                                            float alpha) {
+  const uint4 nb = tab[2 * mk], dc = tab[2 * mk + 1];
+  float val = 0.0f;
+  val += __uint_as_float(__float_as_uint(pw) & nb.x);
+  val += __uint_as_float(__float_as_uint(pe) & nb.y);
+  val += __uint_as_float(__float_as_uint(ps) & nb.z);
+  val += __uint_as_float(__float_as_uint(pn) & nb.w);
+  val += fhh;
+  const float inv = __uint_as_float(dc.x);
+  const float q = val * inv;
+  const float r = fmaf(__uint_as_float(dc.y), q, val);
+  const float q2 = fmaf(r, inv, q);
+  val = __uint_as_float(__float_as_uint(q2) & dc.z);
+  return __uint_as_float(dc.w) * (alpha * val + (1.0f - alpha) * pc);
+}
 
 // a lane's two cells at element alignment: a row starts at any multiple of 4
 // bytes, and gfx950 loads and stores a dword pair at any such address
@@ -72,6 +110,11 @@ template <int NU_, int RPW_, int WAVES_> struct RegTile {
   static constexpr int XBUF = WAVES * 2 * XROW;
   static constexpr size_t LDS = sizeof(uint4) * kRuleEntries + 3 * XBUF * sizeof(float);
 };
+
+// the shapes in use
+template <int NU> using RegTileSmall = RegTile<NU, 2, 16>;
+template <int NU> using RegTileMid = RegTile<NU, 4, 8>;
+template <int NU> using RegTileBig = RegTile<NU, 6, 8>;
 
 // a tile's registers and its place in the level
 template <class T> struct TileRegs {
