@@ -39,7 +39,9 @@ CASES = [  # W, H, smoothing, flags, alpha
     (121, 97, 0, "noise", 1.0),
     (118, 241, 2, "open", 0.8),
     (150, 90, 5, "disks", 1.0),     # more sweeps than a pass holds
-    (1001, 603, 3, "disks", 1.0),   # the middle shape
+    (901, 331, 3, "disks", 1.0),    # the second shape
+    (1000, 421, 2, "noise", 1.0),
+    (1001, 603, 3, "disks", 1.0),   # the third shape
     (1000, 602, 2, "open", 1.0),
     (2101, 1001, 3, "disks", 1.0),  # the large shape
     (2100, 1000, 2, "noise", 1.0),

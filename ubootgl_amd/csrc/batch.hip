@@ -894,19 +894,21 @@ int BatchEngine::build_tiles() {
       ny = cdiv(G.h[l] - 2, PCH);
     });
   }
-  // Level passes: one tile shape per level, by the tuning or by the number of
-  // 128 x 32 regions of its members (the single-domain rule over all of
-  // them); each domain's columns split evenly.
+  // Level passes: one tile shape per pass of a level, by the tuning or by the
+  // members' tiles together; each domain's columns split evenly.
   auto passes = [&](Span *out, bool pre, int nu) {
     for (int l = 0; l < BMAXL && tiled(); l++) {
-      int ox0 = 0, oy0 = 0;
-      pass_tile(PASS_SMALL, true, nu, &ox0, &oy0);
-      long tiles = 0;
-      for (int s = 0; s < nr; s++) {
-        const BGeom &G = *run_[s]->g;
-        if (l < G.cfirst) tiles += (long)cdiv(G.w[l], ox0) * cdiv(G.h[l], oy0);
-      }
-      PassShape shape = tiles <= 256 ? PASS_SMALL : (tiles <= 1024 ? PASS_MID : PASS_BIG);
+      auto tiles = [&](PassShape shape) {
+        int ox = 0, oy = 0;
+        pass_tile(shape, pre, nu, &ox, &oy);
+        long t = 0;
+        for (int s = 0; s < nr; s++) {
+          const BGeom &G = *run_[s]->g;
+          if (l < G.cfirst) t += (long)cdiv(G.w[l], ox) * cdiv(G.h[l], oy);
+        }
+        return t;
+      };
+      PassShape shape = pass_shape(tiles(PASS_TINY), tiles(PASS_SMALL));
       if (tune_.prow) shape = tune_.prow == 8 ? PASS_SMALL : (tune_.prow == 16 ? PASS_MID : PASS_BIG);
       int otx = 0, oty = 0;
       pass_tile(shape, pre, nu, &otx, &oty);

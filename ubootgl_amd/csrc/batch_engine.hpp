@@ -12,6 +12,7 @@
 
 #include "capi_common.hpp"
 #include "coarse_device.hpp"
+#include "regtile_device.hpp"
 
 #include <map>
 #include <memory>
@@ -98,9 +99,6 @@ struct BDomain {
   int cur[BMAXL] = {};
   int xcur = 0;
 };
-
-// tile shapes of the level passes: 16 waves of 2 rows, 8 of 4, 8 of 6
-enum PassShape { PASS_SMALL, PASS_MID, PASS_BIG };
 
 struct Tuning {
   int tx = 64, ty = 8, blocks = 0; // smoother tile (sweep stages), workgroups per launch

@@ -52,34 +52,11 @@ void launch(bool pre, bool zg, int blocks, hipStream_t s, const StageArgs &a) {
   hipLaunchKernelGGL(k, dim3(blocks), dim3(T::TPB), T::LDS, s, a);
 }
 
-template <class Fn> void with_shape(PassShape shape, int nu, Fn fn) {
-  auto by_shape = [&](auto n) {
-    constexpr int NU = decltype(n)::value;
-    if (shape == PASS_SMALL) fn(RegTileSmall<NU>{});
-    else if (shape == PASS_MID) fn(RegTileMid<NU>{});
-    else fn(RegTileBig<NU>{});
-  };
-  switch (nu) {
-  case 0: by_shape(std::integral_constant<int, 0>{}); break;
-  case 1: by_shape(std::integral_constant<int, 1>{}); break;
-  case 2: by_shape(std::integral_constant<int, 2>{}); break;
-  default: by_shape(std::integral_constant<int, 3>{}); break;
-  }
-}
-
 } // namespace
-
-void pass_tile(PassShape shape, bool pre, int nu, int *otx, int *oty) {
-  with_shape(shape, nu, [&](auto t) {
-    using T = decltype(t);
-    *otx = pre ? T::OTXP : T::OTXQ;
-    *oty = pre ? T::OTYP : T::OTYQ;
-  });
-}
 
 void launch_batch_pass(PassShape shape, bool pre, int nu, bool zg, int blocks, hipStream_t s,
                        const StageArgs &a) {
-  with_shape(shape, nu, [&](auto t) { launch<decltype(t)>(pre, zg, blocks, s, a); });
+  with_pass(shape, nu, [&](auto t) { launch<decltype(t)>(pre, zg, blocks, s, a); });
 }
 
 } // namespace ubg

@@ -73,7 +73,6 @@ struct TileWalk {
 // p[ia], writes p[ia^1] and the coarse rhs; post reads p[ia] and the coarse
 // solution p[ib], writes p[ia^1].  Level 0 reads its p and, with zg, takes
 // setZeroGradientBC; the levels below start from zero.
-void pass_tile(PassShape shape, bool pre, int nu, int *otx, int *oty); // largest owned tile
 void launch_batch_pass(PassShape shape, bool pre, int nu, bool zg, int blocks, hipStream_t s,
                        const StageArgs &a);
 

@@ -108,13 +108,93 @@ template <int NU_, int RPW_, int WAVES_> struct RegTile {
   // LDS: rule table, three exchange buffers of two half rows per wave
   static constexpr int XROW = 64;               // floats
   static constexpr int XBUF = WAVES * 2 * XROW;
-  static constexpr size_t LDS = sizeof(uint4) * kRuleEntries + 3 * XBUF * sizeof(float);
+  // HOLD: the smoothing constants of the lane's cells are decoded once into
+  // registers; else rows that are not uniform look them up in LDS per update
+  static constexpr bool HOLD = RPW <= 2;
+  static constexpr size_t TAB = HOLD ? 0 : sizeof(uint4) * kRuleEntries;
+  static constexpr size_t LDS = TAB + 3 * XBUF * sizeof(float);
 };
 
-// the shapes in use
+// a cell's smoothing constants as smooth_tab's table holds them
+struct HeldRule {
+  unsigned w, e, s, n, some; // selectors
+  float inv, ns, F;
+};
+__device__ __forceinline__ HeldRule held_rule(unsigned mk) {
+  HeldRule r;
+  r.w = 0u - ((mk >> 1) & 1u);
+  r.e = 0u - ((mk >> 2) & 1u);
+  r.s = 0u - ((mk >> 3) & 1u);
+  r.n = 0u - ((mk >> 4) & 1u);
+  const unsigned c = mk >> 5;
+  r.inv = c == 3u ? (1.0f / 3.0f) : __int_as_float((int)((127u - (c >> 1)) << 23));
+  r.ns = -(float)c;
+  r.some = c == 0u ? 0u : ~0u;
+  r.F = (float)(mk & MK_SELF);
+  return r;
+}
+__device__ __forceinline__ float smooth_held(float pc, float pw, float pe, float ps, float pn,
+                                             float fhh, const HeldRule &r, float alpha) {
+  float val = 0.0f;
+  val += __uint_as_float(__float_as_uint(pw) & r.w);
+  val += __uint_as_float(__float_as_uint(pe) & r.e);
+  val += __uint_as_float(__float_as_uint(ps) & r.s);
+  val += __uint_as_float(__float_as_uint(pn) & r.n);
+  val += fhh;
+  const float q = val * r.inv;
+  const float q2 = fmaf(fmaf(r.ns, q, val), r.inv, q);
+  val = __uint_as_float(__float_as_uint(q2) & r.some);
+  return r.F * (alpha * val + (1.0f - alpha) * pc);
+}
+
+// The shapes in use, and which a pass takes by the number of tiles its level
+// splits into (the batched solver: its members' tiles together).  Up to one
+// workgroup per CU a launch is all latency, and the shape with the fewest
+// waves whose tiles still fit is the fastest: 12 waves of 2 rows, then 16
+// (256x128 at 3/3: 5.2 + 5.7 us with 12, 5.7 + 6.3 with 16, 7.0 + 7.8 with 8
+// waves of 4 rows; 1090x436 at 2/2: 6.0 + 6.6 us with 16 against 7.1 + 7.7
+// with 12, whose 370 tiles exceed the CUs).  Up to four per CU: 8 waves of 4
+// rows, so that several workgroups share a CU and one loads while another
+// computes (1280x720 at 3/3: 10.4 + 10.0 us against 11.3 + 11.4 us with 8
+// waves of 6 rows and 11.1 + 9.7 us with 16 of 2).  Above: 8 waves of 6 rows,
+// whose halo rows are a smaller share (4096x2048 at 2/2: 33.6 + 31.2 us
+// against 38.5 + 35.5 us with 8 rows, whose fewer workgroups overlap less;
+// 3072x1536 at 3/3: 29.2 + 27.0 us against 32.6 + 28.9 us with 4).
+template <int NU> using RegTileTiny = RegTile<NU, 2, 12>;
 template <int NU> using RegTileSmall = RegTile<NU, 2, 16>;
 template <int NU> using RegTileMid = RegTile<NU, 4, 8>;
 template <int NU> using RegTileBig = RegTile<NU, 6, 8>;
+enum PassShape { PASS_TINY, PASS_SMALL, PASS_MID, PASS_BIG };
+constexpr long kPassCUs = 256;
+// tiny_tiles, small_tiles: tiles of the two small shapes (Mid has as many as Small)
+inline PassShape pass_shape(long tiny_tiles, long small_tiles) {
+  if (tiny_tiles <= kPassCUs) return PASS_TINY;
+  if (small_tiles <= kPassCUs) return PASS_SMALL;
+  return small_tiles <= 4 * kPassCUs ? PASS_MID : PASS_BIG;
+}
+// fn(shape's RegTile<NU>{})
+template <int NU, class Fn> void with_pass_shape(PassShape shape, Fn fn) {
+  if (shape == PASS_TINY) fn(RegTileTiny<NU>{});
+  else if (shape == PASS_SMALL) fn(RegTileSmall<NU>{});
+  else if (shape == PASS_MID) fn(RegTileMid<NU>{});
+  else fn(RegTileBig<NU>{});
+}
+template <class Fn> void with_pass(PassShape shape, int nu, Fn fn) {
+  switch (nu) {
+  case 0: with_pass_shape<0>(shape, fn); break;
+  case 1: with_pass_shape<1>(shape, fn); break;
+  case 2: with_pass_shape<2>(shape, fn); break;
+  default: with_pass_shape<3>(shape, fn); break;
+  }
+}
+// the largest tile a shape's pass owns
+inline void pass_tile(PassShape shape, bool pre, int nu, int *otx, int *oty) {
+  with_pass(shape, nu, [&](auto t) {
+    using T = decltype(t);
+    *otx = pre ? T::OTXP : T::OTXQ;
+    *oty = pre ? T::OTYP : T::OTYQ;
+  });
+}
 
 // a tile's registers and its place in the level
 template <class T> struct TileRegs {
@@ -122,6 +202,7 @@ template <class T> struct TileRegs {
   float P[RPW][CPL], F[RPW][CPL];
   unsigned M[RPW];                 // mask bytes of the lane's cells
   float below[CPL], above[CPL];    // the rows next to the wave's
+  HeldRule rule[T::HOLD ? RPW : 1][CPL];
   const uint4 *tab;
   float *xb;                       // exchange buffers
   int w, h, lane, wave, x0, y0;    // x0: the lane's first column, y0: the wave's first row
@@ -134,7 +215,7 @@ template <class T> struct TileRegs {
 
   __device__ __forceinline__ void place(char *smem, int gx0, int gy0, int w_, int h_) {
     tab = (const uint4 *)smem;
-    xb = (float *)(smem + sizeof(uint4) * kRuleEntries);
+    xb = (float *)(smem + T::TAB);
     w = w_;
     h = h_;
     lane = threadIdx.x & 63;
@@ -192,6 +273,13 @@ template <class T> struct TileRegs {
     ok = __builtin_amdgcn_readfirstlane(ok);
     fast = __builtin_amdgcn_readfirstlane(fast);
     straight = !edge && fast == (1u << RPW) - 1u;
+    if (T::HOLD && !straight) {
+      stay_branch();
+#pragma unroll
+      for (int i = 0; i < (T::HOLD ? RPW : 0); i++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++) rule[i][c] = held_rule(mask_of(i, c));
+    }
   }
 
   __device__ __forceinline__ unsigned mask_of(int i, int c) const { return (M[i] >> (8 * c)) & 0xffu; }
@@ -225,6 +313,18 @@ template <class T> struct TileRegs {
       for (int i = 0; i < RPW; i++)
 #pragma unroll
         for (int c = (S + i) & 1; c < CPL; c += 2) P[i][c] = relaxed(i, c, hh);
+      return;
+    }
+    if (T::HOLD) {
+      stay_branch();
+#pragma unroll
+      for (int i = 0; i < RPW; i++)
+#pragma unroll
+        for (int c = (S + i) & 1; c < CPL; c += 2) {
+          const float v = smooth_held(P[i][c], west(i, c), east(i, c), south(i, c), north(i, c),
+                                      F[i][c] * hh * hh, rule[T::HOLD ? i : 0][c], alpha);
+          P[i][c] = xin[c] && ((ok >> i) & 1u) ? v : P[i][c];
+        }
       return;
     }
 #pragma unroll
@@ -366,8 +466,10 @@ regtile_pre(char *smem, int X0, int Y0, int otx, int oty, const float *__restric
       for (int i = 0; i < RPW; i++) t.P[i][c] = 0.0f;
     }
   }
-  fill_rule_table((uint4 *)smem);
-  __syncthreads();
+  if (!T::HOLD) {
+    fill_rule_table((uint4 *)smem);
+    __syncthreads();
+  }
   if (t.shifted()) {
     stay_branch();
     t.shift_tile(!ZP);
@@ -493,8 +595,10 @@ regtile_post(char *smem, int X0, int Y0, int otx, int oty, const float *__restri
   }
 #pragma unroll
   for (int i = 0; i < RPW; i++) t.load_row(t.F[i], f, t.y0 + i);
-  fill_rule_table((uint4 *)smem);
-  __syncthreads();
+  if (!T::HOLD) {
+    fill_rule_table((uint4 *)smem);
+    __syncthreads();
+  }
   if (t.shifted()) {
     stay_branch();
     t.shift_tile(true);

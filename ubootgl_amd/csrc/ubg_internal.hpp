@@ -88,7 +88,7 @@ void launch_zero_gradient(float *p, int w, int h, hipStream_t s);
 // Level passes (mg_regtile.hip; ping-pong: read L.p, write L.p_alt, swap) of
 // up to kNuPass sweeps:
 //   nu sweeps, residual, restriction into C.  zero_p: L.p is zero on entry
-//   and is not read; zero_coarse: C.p = 0 in the interior (else C.p is left
+//   and is not read (below the finest level: zg is not looked at); zero_coarse: C.p = 0 in the interior (else C.p is left
 //   as it is, for a coarse pass that does not read it);
 constexpr int kNuPass = 3;
 void launch_level_pre(Level &L, Level &C, int nu, float h, float alpha, bool zero_p, bool zg,
