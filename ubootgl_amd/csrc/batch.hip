@@ -592,11 +592,14 @@ int BatchEngine::geom_create(Arena &arena, int W, int H, const float *flag, BGeo
     q += al(n);
   }
   UBG_HIP(hipMemcpyAsync(g->flag[0], f8.data(), f8.size(), hipMemcpyHostToDevice, stream_));
-  launch_build_mask(g->flag[0], g->mask[0], W, H, stream_);
-  for (int l = 1; l < g->nlev; l++) {
-    launch_coarsen(g->flag[l - 1], g->w[l - 1], g->flag[l], g->w[l], g->h[l], stream_);
-    launch_build_mask(g->flag[l], g->mask[l], g->w[l], g->h[l], stream_);
+  std::vector<Level> lv((size_t)g->nlev);
+  for (int l = 0; l < g->nlev; l++) {
+    lv[l].w = g->w[l];
+    lv[l].h = g->h[l];
+    lv[l].flag = g->flag[l];
+    lv[l].mask = g->mask[l];
   }
+  launch_classify(lv.data(), g->nlev, nullptr, false, stream_);
   UBG_TRY(check_launch());
   UBG_HIP(hipStreamSynchronize(stream_)); // f8 is a host temporary
   g->refs = 1;

@@ -252,11 +252,7 @@ struct ubg_mg {
   // coarse flags of levels 1..L-1 from the level-0 flag (updateFields)
   void classify() {
     flag_gen++;
-    launch_build_mask(lv[0].flag, lv[0].mask, lv[0].w, lv[0].h, stream);
-    for (int l = 1; l < levels; l++) {
-      launch_coarsen(lv[l - 1].flag, lv[l - 1].w, lv[l].flag, lv[l].w, lv[l].h, stream);
-      launch_build_mask(lv[l].flag, lv[l].mask, lv[l].w, lv[l].h, stream);
-    }
+    launch_classify(lv.data(), levels, nullptr, false, stream);
   }
 };
 

@@ -68,24 +68,223 @@ __global__ void k_build_mask(const uint8_t *__restrict__ fl, uint8_t *__restrict
   m[i] = (uint8_t)(b | (cnt << 5));
 }
 
-// pressure_solver.hpp:43-56: coarse flag is 1 iff sum(w * f)/16 > 0.2 over the
-// full-weighting stencil; for 0/1 fine flags that is the integer rule
-// weighted count >= 4.  The coarse boundary is 1 (fill(1.0), :41).
-__global__ void k_coarsen(const uint8_t *__restrict__ ff, int wf, uint8_t *__restrict__ fc,
-                          int wc, int hc) {
-  int x = blockIdx.x * blockDim.x + threadIdx.x;
-  int y = blockIdx.y;
-  if (x >= wc) return;
-  uint8_t out = 1;
-  if (x >= 1 && x < wc - 1 && y >= 1 && y < hc - 1) {
-    const uint8_t *r0 = ff + (size_t)(2 * y - 1) * wf + 2 * x;
-    const uint8_t *r1 = r0 + wf;
-    const uint8_t *r2 = r1 + wf;
-    int v = (r0[-1] + 2 * r0[0] + r0[1]) + 2 * (r1[-1] + 2 * r1[0] + r1[1]) +
-            (r2[-1] + 2 * r2[0] + r2[1]);
-    out = v >= 4 ? 1 : 0;
+// Coarse flags and neighbour masks of a hierarchy (updateFields,
+// pressure_solver.hpp:40-57).  pressure_solver.hpp:43-56: coarse flag is 1 iff
+// sum(w * f)/16 > 0.2 over the full-weighting stencil; for 0/1 fine flags that
+// is the integer rule weighted count >= 4.  The coarse boundary is 1
+// (fill(1.0), :41).
+//
+// The flags of level l + 1 need those of level l, so a launch a level (and one
+// more for its mask, and a fill of the coarse fields) leaves a hierarchy's
+// set-up to launch latency: at 1025x1025 20 launches of 2 to 8 us.  Here a
+// workgroup takes a 64x64 tile of a level with the halo that three coarsenings
+// reach (7 cells before it, 4 behind), keeps the flags of all four levels in
+// LDS and writes the tile's masks and coarse flags; a level of at most
+// kClassRest cells and all below it are one workgroup's, bound by its
+// passes' latency.  1025x1025: 8.3 + 14.9 us for two launches instead of 55 us
+// and 18 launch gaps; the allocation-free V-cycle on it 126 -> 96 us.  (A
+// tail from 32x32 cells costs one more launch of the first kind.)
+//
+// Flags are bytes 0 / 1, so four cells' masks are one word: each neighbour's
+// bit and its count (bits 5..7) come from one multiply-add, and no byte of a
+// sum exceeds 159.
+constexpr int CLT = 64;           // cells of a tile
+constexpr int CLP0 = 80, CLH0 = CLT + 11; // first level's LDS rows (words of 4 cells from X0 - 8)
+constexpr int CLR1 = CLT / 2 + 5, CLR2 = CLT / 4 + 2;
+constexpr int kClassThreads = 1024, kClassRest = 16384;
+typedef uint32_t word_u __attribute__((aligned(1)));
+struct ClassStage {
+  const uint8_t *src;     // flags of the first level
+  uint8_t *copy;          // first level's flags as 0 / 1 (null: not written)
+  uint8_t *flag[4], *mask[3];
+  float *zero[4][3];      // fields of the coarse levels to clear (null: none)
+  int w[4], h[4];
+  int n;                  // levels below the first: 0 .. 3
+};
+// masks of one cell or of four, from their flags and their neighbours'
+__device__ __forceinline__ unsigned mask_bytes(unsigned c, unsigned w, unsigned e, unsigned s,
+                                               unsigned n) {
+  static_assert(MK_SELF == 1 && MK_W == 2 && MK_E == 4 && MK_S == 8 && MK_N == 16, "mask bits");
+  return c + w * 34u + e * 36u + s * 40u + n * 48u;
+}
+// coarse flag from the 3x3 fine flags around f (rows of `pitch` bytes)
+__device__ __forceinline__ unsigned coarse_flag(const uint8_t *f, int pitch) {
+  const uint8_t *r0 = f - pitch, *r2 = f + pitch;
+  const int v = (r0[-1] + 2 * r0[0] + r0[1]) + 2 * (f[-1] + 2 * f[0] + f[1]) +
+                (r2[-1] + 2 * r2[0] + r2[1]);
+  return v >= 4 ? 1u : 0u;
+}
+
+__global__ void __launch_bounds__(kClassThreads) k_classify(ClassStage a) {
+  constexpr int PW = CLP0 / 4;
+  __shared__ uint32_t f0_[CLH0 * PW + 2];
+  uint32_t *const f0 = f0_ + 1; // cell (x, y): byte x - X0 + 8 of row y - Y0 + 7
+  __shared__ uint8_t f1[CLR1 * CLR1], f2[CLR2 * CLR2];
+  const int X0 = blockIdx.x * CLT, Y0 = blockIdx.y * CLT, w0 = a.w[0], h0 = a.h[0];
+  constexpr int NLD = (CLH0 * PW + kClassThreads - 1) / kClassThreads;
+  uint32_t v0[NLD];
+#pragma unroll
+  for (int k = 0; k < NLD; k++) {
+    const int i = threadIdx.x + k * kClassThreads;
+    const int x = X0 - 8 + 4 * (i % PW), y = Y0 - 7 + i / PW;
+    v0[k] = 0u;
+    if (y < 0 || y >= h0 || i >= CLH0 * PW) continue;
+    const uint8_t *row = a.src + (size_t)y * w0;
+    if (x >= 0 && x + 4 <= w0) v0[k] = *(const word_u *)(row + x);
+    else
+      for (int c = 0; c < 4; c++)
+        if (x + c >= 0 && x + c < w0) v0[k] |= (uint32_t)row[x + c] << (8 * c);
   }
-  fc[(size_t)y * wc + x] = out;
+#pragma unroll
+  for (int k = 0; k < NLD; k++) {
+    const int i = threadIdx.x + k * kClassThreads;
+    uint32_t t = v0[k]; // bit 0 of a byte: the or of its bits
+    t |= t >> 4;
+    t |= t >> 2;
+    t |= t >> 1;
+    if (i < CLH0 * PW) f0[i] = t & 0x01010101u;
+  }
+  __syncthreads();
+  { // the tile's masks, four cells a thread: 16 words x 64 rows
+    static_assert(CLT / 4 * CLT == kClassThreads, "one word a thread");
+    const int i = threadIdx.x % (CLT / 4), y = threadIdx.x / (CLT / 4), x = X0 + 4 * i;
+    const uint32_t *r = f0 + (y + 7) * PW + i + 2;
+    const uint32_t c = r[0], wst = (c << 8) | (r[-1] >> 24), e = (c >> 8) | (r[1] << 24);
+    const uint32_t m = mask_bytes(c, wst, e, r[-PW], r[PW]);
+    if (Y0 + y < h0) {
+      const size_t o = (size_t)(Y0 + y) * w0 + x;
+      if (x + 4 <= w0) {
+        *(word_u *)(a.mask[0] + o) = m;
+        if (a.copy) *(word_u *)(a.copy + o) = c;
+      } else
+        for (int k = 0; k < 4; k++)
+          if (x + k < w0) {
+            a.mask[0][o + k] = (uint8_t)(m >> (8 * k));
+            if (a.copy) a.copy[o + k] = (uint8_t)(c >> (8 * k));
+          }
+    }
+  }
+  // cell (x, y) of the stage's level k with flag v, in LDS region r x r from
+  // (x0, y0); the tile owns t x t cells from (x0 + lo, y0 + lo)
+  auto put = [&](int k, int x, int y, unsigned v, uint8_t *out, int r, int lo, int t) {
+    const int rx = x - ((X0 >> k) - lo), ry = y - ((Y0 >> k) - lo), w = a.w[k], h = a.h[k];
+    if (rx < 0 || rx >= r || ry < 0 || ry >= r) return;
+    const bool in = x >= 0 && x < w && y >= 0 && y < h;
+    if (!in) v = 0;
+    else if (x == 0 || x == w - 1 || y == 0 || y == h - 1) v = 1;
+    if (out) out[ry * r + rx] = (uint8_t)v;
+    if (in && rx >= lo && rx < lo + t && ry >= lo && ry < lo + t) {
+      const size_t o = (size_t)y * w + x;
+      a.flag[k][o] = (uint8_t)v;
+      if (a.zero[k][0]) a.zero[k][0][o] = a.zero[k][1][o] = a.zero[k][2][o] = 0.0f;
+    }
+  };
+  auto masks = [&](int k, const uint8_t *f, int r, int lo, int t) {
+    for (int i = threadIdx.x; i < t * t; i += kClassThreads) {
+      const int x = i % t, y = i / t, gx = (X0 >> k) + x, gy = (Y0 >> k) + y;
+      if (gx >= a.w[k] || gy >= a.h[k]) continue;
+      const uint8_t *q = f + (y + lo) * r + x + lo;
+      a.mask[k][(size_t)gy * a.w[k] + gx] =
+          (uint8_t)mask_bytes(q[0], q[-1], q[1], q[-r], q[r]);
+    }
+  };
+  if (a.n < 1) return;
+  // level 1, two cells of a row from a word: the column sums of its three
+  // rows, then each byte with its neighbours (at most 16).  The first cell of
+  // word 0 lies outside the region.
+  if (threadIdx.x < CLR1 * (PW - 1)) {
+    const int i = threadIdx.x % (PW - 1), ry = threadIdx.x / (PW - 1);
+    const int y = (Y0 >> 1) - 3 + ry, x = (X0 - 8 + 4 * i) >> 1; // cells x, x + 1
+    const uint32_t *r = f0 + (2 * ry + 1) * PW + i;              // row 2 y
+    auto column = [&](int d) { return r[d - PW] + 2u * r[d] + r[d + PW]; };
+    const uint32_t c = column(0), l = (c << 8) | (column(-1) >> 24);
+    const uint32_t t = l + 2u * c + (c >> 8); // bytes 0 and 2 are whole
+    put(1, x, y, (t & 0xffu) >= 4u, f1, CLR1, 3, CLT / 2);
+    put(1, x + 1, y, ((t >> 16) & 0xffu) >= 4u, f1, CLR1, 3, CLT / 2);
+  }
+  __syncthreads();
+  masks(1, f1, CLR1, 3, CLT / 2);
+  if (a.n < 2) return;
+  if (threadIdx.x < CLR2 * CLR2) {
+    const int rx = threadIdx.x % CLR2, ry = threadIdx.x / CLR2;
+    put(2, (X0 >> 2) - 1 + rx, (Y0 >> 2) - 1 + ry,
+        coarse_flag(f1 + (2 * ry + 1) * CLR1 + 2 * rx + 1, CLR1), f2, CLR2, 1, CLT / 4);
+  }
+  __syncthreads();
+  masks(2, f2, CLR2, 1, CLT / 4);
+  if (a.n < 3) return;
+  if (threadIdx.x < CLT / 8 * (CLT / 8)) {
+    const int rx = threadIdx.x % (CLT / 8), ry = threadIdx.x / (CLT / 8);
+    put(3, (X0 >> 3) + rx, (Y0 >> 3) + ry,
+        coarse_flag(f2 + (2 * ry + 1) * CLR2 + 2 * rx + 1, CLR2), nullptr, CLT / 8, 0, CLT / 8);
+  }
+}
+
+// the level of at most kClassRest cells and all below it: level k's flags in
+// one LDS buffer, level k + 1's into the other, each with a ring of zeros
+struct ClassRest {
+  const uint8_t *src;
+  uint8_t *copy;
+  uint8_t *flag[16], *mask[16];
+  float *zero[16][3];
+  int w[16], h[16];
+  int n; // levels below the first
+};
+constexpr int kClassRing = kClassRest + 2 * (kClassRest / 4 + 4) + 4; // (w + 2)(h + 2), w, h >= 4
+__global__ void __launch_bounds__(1024) k_classify_rest(ClassRest a) {
+  __shared__ uint8_t buf[2][kClassRing];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // rings: the cells of a level are written between the barriers
+  auto ring = [&](uint8_t *f, int w, int h) {
+    for (int i = threadIdx.x; i < w + 2; i += 1024) f[i] = f[(h + 1) * (w + 2) + i] = 0;
+    for (int i = threadIdx.x; i < h; i += 1024) f[(i + 1) * (w + 2)] = f[(i + 2) * (w + 2) - 1] = 0;
+  };
+  const int w0 = a.w[0], h0 = a.h[0];
+  ring(buf[0], w0, h0);
+  for (int x = lane; x < w0; x += 64)
+    for (int y = wave; y < h0; y += 16 * 8) { // eight loads in flight
+      uint8_t v[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] = a.src[min(y + 16 * j, h0 - 1) * w0 + x];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        if (y + 16 * j >= h0) break;
+        v[j] = v[j] != 0 ? 1 : 0;
+        buf[0][(y + 16 * j + 1) * (w0 + 2) + x + 1] = v[j];
+        if (a.copy) a.copy[(y + 16 * j) * w0 + x] = v[j];
+      }
+    }
+  __syncthreads();
+  for (int k = 0;; k++) {
+    const int w = a.w[k], h = a.h[k], p = w + 2;
+    const uint8_t *f = buf[k & 1] + p + 1; // cell (0, 0)
+    uint8_t *const mask = a.mask[k];
+    for (int x = lane; x < w; x += 64)
+#pragma unroll 4
+      for (int y = wave; y < h; y += 16) {
+        const uint8_t *q = f + y * p + x;
+        mask[y * w + x] = (uint8_t)mask_bytes(q[0], q[-1], q[1], q[-p], q[p]);
+      }
+    if (k == a.n) return;
+    const int wc = a.w[k + 1], hc = a.h[k + 1];
+    uint8_t *c = buf[(k + 1) & 1];
+    ring(c, wc, hc);
+    c += wc + 3;
+    uint8_t *const flag = a.flag[k + 1];
+    float *const z0 = a.zero[k + 1][0], *const z1 = a.zero[k + 1][1], *const z2 = a.zero[k + 1][2];
+    for (int x = lane; x < wc; x += 64)
+#pragma unroll 2
+      for (int y = wave; y < hc; y += 16) {
+        const int i = y * wc + x;
+        const unsigned v = x == 0 || x == wc - 1 || y == 0 || y == hc - 1
+                               ? 1u
+                               : coarse_flag(f + 2 * y * p + 2 * x, p);
+        c[y * (wc + 2) + x] = (uint8_t)v;
+        flag[i] = (uint8_t)v;
+        if (z0) z0[i] = z1[i] = z2[i] = 0.0f;
+      }
+    __syncthreads();
+  }
 }
 
 // setZeroGradientBC (pressure_solver.cpp:183-192): edges copy the first
@@ -283,8 +482,50 @@ void launch_sumsq(const float *src, size_t n, double *acc, hipStream_t s) {
 void launch_build_mask(const uint8_t *flag, uint8_t *mask, int w, int h, hipStream_t s) {
   hipLaunchKernelGGL(k_build_mask, dim3(ceil_div(w, TPB), h), dim3(TPB), 0, s, flag, mask, w, h);
 }
-void launch_coarsen(const uint8_t *ff, int wf, uint8_t *fc, int wc, int hc, hipStream_t s) {
-  hipLaunchKernelGGL(k_coarsen, dim3(ceil_div(wc, TPB), hc), dim3(TPB), 0, s, ff, wf, fc, wc, hc);
+void launch_classify(const Level *lv, int levels, const uint8_t *raw, bool zero, hipStream_t s) {
+  int l = 0;
+  const uint8_t *src = raw ? raw : lv[0].flag;
+  uint8_t *copy = raw ? lv[0].flag : nullptr;
+  for (; (size_t)lv[l].w * lv[l].h > kClassRest; l += 3) {
+    ClassStage a{};
+    a.src = src;
+    a.copy = copy;
+    a.n = levels - 1 - l < 3 ? levels - 1 - l : 3;
+    for (int k = 0; k <= a.n; k++) {
+      const Level &L = lv[l + k];
+      a.w[k] = L.w;
+      a.h[k] = L.h;
+      a.flag[k] = L.flag;
+      if (k < 3) a.mask[k] = L.mask;
+      if (zero && k > 0) {
+        a.zero[k][0] = L.p;
+        a.zero[k][1] = L.p_alt;
+        a.zero[k][2] = L.f;
+      }
+    }
+    hipLaunchKernelGGL(k_classify, dim3(ceil_div(lv[l].w, CLT), ceil_div(lv[l].h, CLT)),
+                       dim3(kClassThreads), 0, s, a);
+    if (l + 3 > levels - 1) return; // the last level's mask is written
+    src = lv[l + 3].flag;
+    copy = nullptr;
+  }
+  ClassRest a{};
+  a.src = src;
+  a.copy = copy;
+  a.n = levels - 1 - l;
+  for (int k = 0; k <= a.n; k++) {
+    const Level &L = lv[l + k];
+    a.w[k] = L.w;
+    a.h[k] = L.h;
+    a.flag[k] = L.flag;
+    a.mask[k] = L.mask;
+    if (zero && k > 0) {
+      a.zero[k][0] = L.p;
+      a.zero[k][1] = L.p_alt;
+      a.zero[k][2] = L.f;
+    }
+  }
+  hipLaunchKernelGGL(k_classify_rest, dim3(1), dim3(1024), 0, s, a);
 }
 void launch_zero_gradient(float *p, int w, int h, hipStream_t s) {
   int n = w > h ? w : h;

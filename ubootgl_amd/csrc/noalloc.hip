@@ -21,12 +21,6 @@ namespace {
 
 __device__ __align__(256) char scratch[UBG_NOALLOC_SCRATCH_BYTES];
 
-// flags as 0/1 bytes (any nonzero byte is fluid)
-__global__ void k_flag_01(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i] != 0 ? 1 : 0;
-}
-
 struct DeviceScratch {
   char *base = nullptr; // device address of `scratch` on this device
   ubg_mg mg;            // host-side level table, reused by every call
@@ -120,13 +114,11 @@ extern "C" UBG_API int ubg_mg_solve_device_noalloc(float *p, const float *f, con
     L.flag = (uint8_t *)take(n);
     L.mask = (uint8_t *)take(n);
   }
-  // a fresh hierarchy: zero everything this call uses (a fill kernel, no
-  // memset node under capture), then the flags and the coarse classification
-  launch_fill_f32((float *)base, off / 4, 0.0f, s);
+  // a fresh hierarchy: the flags, masks and coarse classification, and zero
+  // coarse fields (level 0's second buffer is written whole before it is read)
+  m.flag_gen++;
+  launch_classify(m.lv.data(), nl, flag, true, s);
   const size_t n0 = (size_t)width * height;
-  hipLaunchKernelGGL(k_flag_01, dim3((unsigned)((n0 + 255) / 256)), dim3(256), 0, s, flag,
-                     m.lv[0].flag, n0);
-  m.classify();
   for (int c = 0; c < ncycles; c++) m.solve_level(0, h, zero_gradient_bc != 0);
   // the sweeps ping-pong between p and p_alt: the result may sit in scratch
   if (m.lv[0].p != p)

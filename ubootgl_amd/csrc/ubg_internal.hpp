@@ -79,7 +79,10 @@ void launch_sumsq(const float *src, size_t n, double *acc, hipStream_t s);
 
 // ---- multigrid (pressure_solver.hpp / pressure_solver.cpp) ---------------
 void launch_build_mask(const uint8_t *flag, uint8_t *mask, int w, int h, hipStream_t s);
-void launch_coarsen(const uint8_t *ff, int wf, uint8_t *fc, int wc, int hc, hipStream_t s);
+// masks of all levels and flags of the coarse ones from level 0's flags, or
+// from `raw` (any nonzero byte is fluid), which level 0's flags are then set
+// from; zero: p, p_alt and f of the coarse levels are cleared
+void launch_classify(const Level *lv, int levels, const uint8_t *raw, bool zero, hipStream_t s);
 // one red+black sweep fused in one launch (streaming waves, ping-pong: reads
 // L.p, writes L.p_alt, then swaps the two pointers); zero_gradient applies
 // setZeroGradientBC to the result.
