@@ -15,6 +15,7 @@
 // skipped on the device; no host round trip is needed per stage.
 #include "batch_stage.hpp"
 #include "mg_device.hpp"
+#include "refine_device.hpp"
 
 #include <algorithm>
 #include <array>
@@ -222,6 +223,7 @@ __device__ __forceinline__ double wsum(double v) {
 // The refinement update of refine.hip's k_ir_update for 256 x 8 tiles of
 // every domain: ia = e index of level 0; ib bit 0 = x index, bit 1 = add e.
 __global__ void __launch_bounds__(B_UPD_W) kb_update(StageArgs a) {
+  static_assert(B_UPD_W == kIrCols && B_UPD_H == kIrRows, "blocks of ir_update_column");
   __shared__ double red[B_UPD_W / 64];
   TileWalk tw;
   if (!tw.init(a)) return;
@@ -242,33 +244,8 @@ __global__ void __launch_bounds__(B_UPD_W) kb_update(StageArgs a) {
     const int w = D.w, h = D.h;
     const double ihsq = 1.0 / ((double)L0.hh * (double)L0.hh);
     const int x = T.x0 + threadIdx.x;
-    const int y0 = T.y0, y1 = min(y0 + B_UPD_H, h);
-    double acc = 0.0;
-    if (x < w) {
-      auto X = [&](size_t i) { return ACC ? xa[i] + (double)e[i] : xa[i]; };
-      size_t c = (size_t)y0 * w + x;
-      double xs = y0 > 0 ? X(c - w) : 0.0;
-      double xc = X(c);
-      for (int y = y0; y < y1; y++, c += w) {
-        const double xn = y + 1 < h ? X(c + w) : 0.0;
-        xb[c] = xc;
-        ez[c] = 0.0f;
-        double r = 0.0;
-        const unsigned mk = m[c];
-        if (x >= 1 && x <= w - 2 && y >= 1 && y <= h - 2 && (mk & MK_SELF)) {
-          double s = 0.0;
-          if (mk & MK_W) s += X(c - 1) - xc;
-          if (mk & MK_E) s += X(c + 1) - xc;
-          if (mk & MK_S) s += xs - xc;
-          if (mk & MK_N) s += xn - xc;
-          r = (double)f[c] + s * ihsq;
-        }
-        r32[c] = (float)r;
-        acc += r * r;
-        xs = xc;
-        xc = xn;
-      }
-    }
+    double acc = ACC ? ir_update_column<true>(x, T.y0, xa, xb, e, ez, f, m, r32, w, h, ihsq)
+                     : ir_update_column<false>(x, T.y0, xa, xb, e, ez, f, m, r32, w, h, ihsq);
     acc = wsum(acc);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
@@ -290,8 +267,7 @@ __global__ void __launch_bounds__(1024) kb_norm(StageArgs a, int nslots) {
   const BDom &D = a.dom[d];
   if (!dom_active(D)) return;
   const int n = D.gx * D.gy;
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) s += D.partial[i];
+  double s = thread_partials(D.partial, n);
   __shared__ double red[16];
   s = wsum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;

@@ -17,6 +17,7 @@
 // HBM bytes per fine cell of the fused pass: x64 read 8 + e32 read 4 +
 // f32 read 4 + mask 1 + x64 write 8 + r32 write 4 + e32 zero 4 = 33.
 #include "capi_common.hpp"
+#include "refine_device.hpp"
 
 struct IRState {
   char *base = nullptr;
@@ -31,51 +32,22 @@ struct IRState {
 namespace ubg {
 namespace {
 
-constexpr int IR_TPB = 256; // cells of one row per block
-constexpr int IR_ROWS = 8;  // rows per block
+constexpr int IR_TPB = kIrCols;  // cells of one row per block
+constexpr int IR_ROWS = kIrRows; // rows per block
 
 __device__ __forceinline__ double warp_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
-// x_b = x_a + e (ACC) or x_a, r32 = (float) r(x_b), e_zero = 0, and one
-// partial sum of r^2 per block.  Neighbour values x_a(n) + e(n) are formed
-// from the inputs, so no thread reads a value another thread writes.
+// one block of the update (refine_device.hpp) and its partial sum of r^2
 template <bool ACC>
 __global__ void __launch_bounds__(IR_TPB)
 k_ir_update(const double *__restrict__ xa, double *__restrict__ xb, const float *__restrict__ e,
             float *__restrict__ ez, const float *__restrict__ f, const uint8_t *__restrict__ m,
             float *__restrict__ r32, int w, int h, double ihsq, double *__restrict__ partial) {
-  const int x = blockIdx.x * IR_TPB + threadIdx.x;
-  const int y0 = blockIdx.y * IR_ROWS;
-  const int y1 = min(y0 + IR_ROWS, h);
-  double acc = 0.0;
-  if (x < w) {
-    auto X = [&](size_t i) { return ACC ? xa[i] + (double)e[i] : xa[i]; };
-    size_t c = (size_t)y0 * w + x;
-    double xs = y0 > 0 ? X(c - w) : 0.0; // row y-1
-    double xc = X(c);
-    for (int y = y0; y < y1; y++, c += w) {
-      const double xn = y + 1 < h ? X(c + w) : 0.0;
-      xb[c] = xc;
-      ez[c] = 0.0f;
-      double r = 0.0;
-      const unsigned mk = m[c];
-      if (x >= 1 && x <= w - 2 && y >= 1 && y <= h - 2 && (mk & MK_SELF)) {
-        double s = 0.0;
-        if (mk & MK_W) s += X(c - 1) - xc;
-        if (mk & MK_E) s += X(c + 1) - xc;
-        if (mk & MK_S) s += xs - xc;
-        if (mk & MK_N) s += xn - xc;
-        r = (double)f[c] + s * ihsq;
-      }
-      r32[c] = (float)r;
-      acc += r * r;
-      xs = xc;
-      xc = xn;
-    }
-  }
+  double acc = ir_update_column<ACC>(blockIdx.x * IR_TPB + threadIdx.x, blockIdx.y * IR_ROWS, xa,
+                                     xb, e, ez, f, m, r32, w, h, ihsq);
   __shared__ double red[IR_TPB / 64];
   acc = warp_sum(acc);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
@@ -90,8 +62,7 @@ k_ir_update(const double *__restrict__ xa, double *__restrict__ xb, const float 
 // out = sum of n partials, one block, fixed order
 __global__ void __launch_bounds__(1024) k_sum_partials(const double *__restrict__ p, int n,
                                                          double *__restrict__ out) {
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) s += p[i];
+  double s = thread_partials(p, n);
   __shared__ double red[16];
   s = warp_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
