@@ -179,6 +179,105 @@ __global__ void k_accumulate(float *__restrict__ xf, float *__restrict__ xa,
 
 __device__ __forceinline__ float fbit(unsigned m, int k) { return ((m >> k) & 1u) ? 1.0f : 0.0f; }
 
+// ---- order of blocks --------------------------------------------------------
+// Blocks go round-robin over the 8 XCDs, so in launch order the rows above and
+// below a block's are read through other L2s.  Diffuse and correction with one
+// cell a lane give each XCD one eighth of the grid in a piece: 1090x436 7.4 ->
+// 5.6 and 6.5 -> 5.5 us, 1921x1081 12.0 -> 12.2 and 13.9 -> 12.3.  (Divergence,
+// which reads each value at most twice, and advect, bound by arithmetic, keep
+// the launch order: no gain, and 1 - 2 us more for a 1921x1081 step.)
+struct BlockXY {
+  int x, y;
+};
+__device__ __forceinline__ BlockXY xcd_block() {
+  const int gx = gridDim.x, b = xcd_tile(blockIdx.y * gx + blockIdx.x, gx * gridDim.y);
+  return BlockXY{b % gx, b / gx};
+}
+
+// ---- wide rows --------------------------------------------------------------
+// On large fields the per-cell passes around the V-cycle (diffuse, setVBCs +
+// divergence, correction) take two cells a lane: a wave has 128 cells of one
+// row from x = 124 s - 2; lanes 0 and 63 are halo, so that the values left and
+// right of a lane's pair come by DPP lane shifts.  The XCDs take turns at
+// bands of WIDE_BAND blocks' rows (gridDim.y is a multiple of 8 WIDE_BAND;
+// blocks beyond the last row end at once), so that all of them work on one
+// part of memory.  See wide_rows for where and the figures.
+constexpr int WIDE = 124, WIDE_WAVES = 4; // cells a wave owns; waves of a block, one row each
+constexpr int WIDE_BAND = 4, WIDE_DIFFUSE = 2; // diffuse: rows of a wave
+static_assert(64 * WIDE_WAVES == TPB, "the launches' block");
+typedef float pair_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t mpair_u __attribute__((aligned(2)));
+struct WideRow {
+  int y;        // the wave's row (0: none)
+  int x;        // the lane's first cell
+  bool own;     // the lane's cells are the wave's
+  bool whole;   // uniform: every cell of the wave has x in 0 .. W - 2
+  bool inner;   // uniform: no cell of the wave has boundary duties
+  __device__ __forceinline__ WideRow(int W, int H, int rows = 1) {
+    const int gx = gridDim.x, b = blockIdx.y * gx + blockIdx.x, slot = b >> 3;
+    const int r = slot / gx, s = slot % gx, lane = threadIdx.x & 63;
+    const int by = (r / WIDE_BAND * 8 + (b & 7)) * WIDE_BAND + r % WIDE_BAND;
+    y = 1 + rows * (by * WIDE_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    y = y <= H - 2 ? y : 0;
+    const int x0 = WIDE * s - 2;
+    x = x0 + 2 * lane;
+    own = lane >= 1 && lane <= 62;
+    whole = s > 0 && x0 + 127 <= W - 2;
+    inner = s > 0 && x0 + 127 < W - 3 && y > 1 && y + rows - 1 < H - 3;
+  }
+  // the lane's pair of row yy of a grid w wide (beyond it some value of the
+  // row); WHOLE: this->whole.  A pass branches once, around all its loads: a
+  // branch in each makes the wave wait for one before the next.
+  template <bool WHOLE>
+  __device__ __forceinline__ void load(float (&v)[2], const float *__restrict__ g, int w,
+                                       int yy) const {
+    const float *row = g + (size_t)yy * w;
+    if (WHOLE) {
+      const pair_u q = *(const pair_u *)((const char *)row + 4u * (unsigned)x);
+      v[0] = q[0];
+      v[1] = q[1];
+    } else {
+      v[0] = row[min(max(x, 0), w - 1)];
+      v[1] = row[min(max(x + 1, 0), w - 1)];
+    }
+  }
+  template <bool WHOLE>
+  __device__ __forceinline__ void load(unsigned (&m)[2], const uint16_t *__restrict__ g, int w,
+                                       int yy) const {
+    const uint16_t *row = g + (size_t)yy * w;
+    if (WHOLE) {
+      const unsigned q = *(const mpair_u *)((const char *)row + 2u * (unsigned)x);
+      m[0] = q & 0xffffu;
+      m[1] = q >> 16;
+    } else {
+      m[0] = row[min(max(x, 0), w - 1)];
+      m[1] = row[min(max(x + 1, 0), w - 1)];
+    }
+  }
+  // fn<WHOLE>(): a pass's loads
+  template <class Fn> __device__ __forceinline__ void loads(Fn fn) const {
+    if (whole) fn(std::true_type{});
+    else fn(std::false_type{});
+  }
+  // the wave's cells with 1 <= x <= last
+  __device__ __forceinline__ bool owns(int xx, int last) const {
+    return own && xx >= 1 && xx <= last;
+  }
+  __device__ __forceinline__ void store(float *__restrict__ g, int w, const float (&v)[2],
+                                        int last, int j = 0) const {
+    float *row = g + (size_t)(y + j) * w;
+    if (owns(x, last) && owns(x + 1, last)) {
+      pair_u q;
+      q[0] = v[0];
+      q[1] = v[1];
+      *(pair_u *)((char *)row + 4u * (unsigned)x) = q;
+    } else {
+      if (owns(x, last)) row[x] = v[0];
+      if (owns(x + 1, last)) row[x + 1] = v[1];
+    }
+  }
+};
+
 __global__ void k_face_masks(const uint8_t *__restrict__ fl, uint16_t *__restrict__ fm, int W,
                              int H) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -221,36 +320,34 @@ __device__ __forceinline__ void diffuse_cell(int x, int y, const float *__restri
                                              float a, const BCGrid &gx, const BCGrid &gy) {
   const int Wx = W - 1, Hy = H - 1;
   if (x >= W - 1) return;
+  const bool hx = x < Wx - 1, hy = y < Hy - 1; // the thread owns a vx / vy face
+  const size_t i = (size_t)y * Wx + (hx ? x : x - 1), k = (size_t)(hy ? y : y - 1) * W + x;
   const unsigned m = fm[(size_t)y * W + x];
+  const float xc = sx[i], xe = sx[i + 1], xw = sx[i - 1], xn = sx[i + Wx], xs = sx[i - Wx];
+  const float yc = sy[k], ys = sy[k - W], yn = sy[k + W], ye = sy[k + 1], yw = sy[k - 1];
   float vxn = 0.0f, vyn = 0.0f;
-  if (x < Wx - 1) {
-    const float *s = sx;
-    size_t i = (size_t)y * Wx + x;
-    float vc = s[i];
+  {
     float val = 0.0f;
-    val += s[i + 1] * fbit(m, 1);
-    val += s[i - 1] * fbit(m, 2);
+    val += xe * fbit(m, 1);
+    val += xw * fbit(m, 2);
     float fvn = fbit(m, 3);
-    val += s[i + Wx] * fvn + (1.0f - fvn) * -vc;
+    val += xn * fvn + (1.0f - fvn) * -xc;
     float fvs = fbit(m, 4);
-    val += s[i - Wx] * fvs + (1.0f - fvs) * -vc;
-    vxn = fbit(m, 0) * (vc + a * val) / (1.0f + 4.0f * a);
-    dx[i] = vxn;
+    val += xs * fvs + (1.0f - fvs) * -xc;
+    vxn = fbit(m, 0) * (xc + a * val) / (1.0f + 4.0f * a);
   }
-  if (y < Hy - 1) {
-    const float *s = sy;
-    size_t i = (size_t)y * W + x;
-    float vc = s[i];
+  {
     float val = 0.0f;
-    val += s[i - W] * fbit(m, 9);
-    val += s[i + W] * fbit(m, 10);
+    val += ys * fbit(m, 9);
+    val += yn * fbit(m, 10);
     float fve = fbit(m, 11);
-    val += s[i + 1] * fve + (1.0f - fve) * -vc;
+    val += ye * fve + (1.0f - fve) * -yc;
     float fvw = fbit(m, 12);
-    val += s[i - 1] * fvw + (1.0f - fvw) * -vc;
-    vyn = fbit(m, 8) * (vc + a * val) / (1.0f + 4.0f * a);
-    dy[i] = vyn;
+    val += yw * fvw + (1.0f - fvw) * -yc;
+    vyn = fbit(m, 8) * (yc + a * val) / (1.0f + 4.0f * a);
   }
+  if (hx) dx[i] = vxn;
+  if (hy) dy[k] = vyn;
   if (x == 1 || x >= W - 3 || y == 1 || y >= H - 3) { // boundary duties
     if (x < Wx - 1) bc_duty(gx, x, y, vxn, nullptr);
     if (y < Hy - 1) bc_duty(gy, x, y, vyn, nullptr);
@@ -260,8 +357,76 @@ __global__ void k_diffuse_both(const float *__restrict__ sx, float *__restrict__
                                const float *__restrict__ sy, float *__restrict__ dy,
                                const uint16_t *__restrict__ fm, int W, int H, float a,
                                BCGrid gx, BCGrid gy) {
-  diffuse_cell(blockIdx.x * blockDim.x + threadIdx.x + 1, blockIdx.y + 1, sx, dx, sy, dy, fm, W, H,
+  const BlockXY b = xcd_block();
+  diffuse_cell(b.x * blockDim.x + threadIdx.x + 1, b.y + 1, sx, dx, sy, dy, fm, W, H,
                a, gx, gy);
+}
+
+// the same on wide rows, two of them a wave
+__global__ void __launch_bounds__(64 * WIDE_WAVES)
+    k_diffuse_wide(const float *__restrict__ sx, float *__restrict__ dx,
+                   const float *__restrict__ sy, float *__restrict__ dy,
+                   const uint16_t *__restrict__ fm, int W, int H, float a, BCGrid gx, BCGrid gy) {
+  constexpr int R = WIDE_DIFFUSE;
+  const WideRow S(W, H, R);
+  const int Wx = W - 1, Hy = H - 1;
+  if (S.y == 0) return;
+  float X[R + 2][2], Y[R + 2][2];
+  unsigned m[R][2];
+  S.loads([&](auto whole) {
+    constexpr bool K = decltype(whole)::value;
+#pragma unroll
+    for (int j = 0; j < R + 2; j++) {
+      S.template load<K>(X[j], sx, Wx, min(S.y - 1 + j, H - 1));
+      S.template load<K>(Y[j], sy, W, min(S.y - 1 + j, Hy - 1));
+    }
+#pragma unroll
+    for (int j = 0; j < R; j++) S.template load<K>(m[j], fm, W, min(S.y + j, H - 2));
+  });
+#pragma unroll
+  for (int j = 0; j < R; j++) {
+    const int y = S.y + j;
+    if (y > H - 2) break;
+    const float xw = from_left(X[j + 1][1]), xe = from_right(X[j + 1][0]);
+    const float yw = from_left(Y[j + 1][1]), ye = from_right(Y[j + 1][0]);
+    float nx[2], ny[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const unsigned k = m[j][c];
+      {
+        const float vc = X[j + 1][c];
+        float val = 0.0f;
+        val += (c ? xe : X[j + 1][1]) * fbit(k, 1);
+        val += (c ? X[j + 1][0] : xw) * fbit(k, 2);
+        const float fvn = fbit(k, 3);
+        val += X[j + 2][c] * fvn + (1.0f - fvn) * -vc;
+        const float fvs = fbit(k, 4);
+        val += X[j][c] * fvs + (1.0f - fvs) * -vc;
+        nx[c] = fbit(k, 0) * (vc + a * val) / (1.0f + 4.0f * a);
+      }
+      {
+        const float vc = Y[j + 1][c];
+        float val = 0.0f;
+        val += Y[j][c] * fbit(k, 9);
+        val += Y[j + 2][c] * fbit(k, 10);
+        const float fve = fbit(k, 11);
+        val += (c ? ye : Y[j + 1][1]) * fve + (1.0f - fve) * -vc;
+        const float fvw = fbit(k, 12);
+        val += (c ? Y[j + 1][0] : yw) * fvw + (1.0f - fvw) * -vc;
+        ny[c] = fbit(k, 8) * (vc + a * val) / (1.0f + 4.0f * a);
+      }
+    }
+    S.store(dx, Wx, nx, Wx - 2, j);
+    if (y < Hy - 1) S.store(dy, W, ny, W - 2, j);
+    if (S.inner) continue;
+#pragma unroll
+    for (int c = 0; c < 2; c++) { // boundary duties
+      const int x = S.x + c;
+      if (!S.owns(x, W - 2)) continue;
+      if (x < Wx - 1) bc_duty(gx, x, y, nx[c], nullptr);
+      if (y < Hy - 1) bc_duty(gy, x, y, ny[c], nullptr);
+    }
+  }
 }
 
 // CubicHermite (interpolators.hpp:78-85), Catmull-Rom, evaluated as
@@ -664,8 +829,53 @@ __global__ void k_correct_tail(float *__restrict__ xf, float *__restrict__ yf,
                                float *__restrict__ p, const uint16_t *__restrict__ fm, int W,
                                int H, float ih, BCGrid gx, BCGrid gy, float *__restrict__ xcur,
                                float *__restrict__ ycur, int bw, int be, int bn, int bs) {
-  correct_tail_cell(blockIdx.x * blockDim.x + threadIdx.x + 1, blockIdx.y + 1, xf, yf, p, fm, W,
+  const BlockXY b = xcd_block();
+  correct_tail_cell(b.x * blockDim.x + threadIdx.x + 1, b.y + 1, xf, yf, p, fm, W,
                     H, ih, gx, gy, xcur, ycur, bw, be, bn, bs);
+}
+
+// the same on wide rows
+__global__ void __launch_bounds__(64 * WIDE_WAVES)
+    k_correct_tail_wide(float *__restrict__ xf, float *__restrict__ yf, float *__restrict__ p,
+                        const uint16_t *__restrict__ fm, int W, int H, float ih, BCGrid gx,
+                        BCGrid gy, float *__restrict__ xcur, float *__restrict__ ycur, int bw,
+                        int be, int bn, int bs) {
+  const WideRow S(W, H);
+  const int Wx = W - 1, y = S.y;
+  if (y == 0) return;
+  const bool hy = y < H - 2; // the row has vy faces
+  float P[2], pn[2], ux[2], uy[2];
+  unsigned m[2]; // F(x)F(x+1) (bit 0) and F(y)F(y+1) (bit 8)
+  S.loads([&](auto whole) {
+    constexpr bool K = decltype(whole)::value;
+    S.template load<K>(P, p, W, y);
+    S.template load<K>(pn, p, W, hy ? y + 1 : y);
+    S.template load<K>(ux, xf, Wx, y);
+    S.template load<K>(uy, yf, W, hy ? y : y - 1);
+    S.template load<K>(m, fm, W, y);
+  });
+  const float pe = from_right(P[0]);
+  float vx[2], vy[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    vx[c] = ux[c] - fbit(m[c], 0) * ih * ((c ? pe : P[1]) - P[c]);
+    vy[c] = uy[c] - fbit(m[c], 8) * ih * (pn[c] - P[c]);
+  }
+  S.store(xf, Wx, vx, W - 3);
+  if (xcur) S.store(xcur, Wx, vx, W - 3);
+  if (hy) {
+    S.store(yf, W, vy, W - 2);
+    if (ycur) S.store(ycur, W, vy, W - 2);
+  }
+  if (S.inner) return;
+#pragma unroll
+  for (int c = 0; c < 2; c++) { // boundary duties
+    const int x = S.x + c;
+    if (!S.owns(x, W - 2)) continue;
+    if (x < W - 2) bc_duty(gx, x, y, vx[c], xcur);
+    if (hy) bc_duty(gy, x, y, vy[c], ycur);
+    pbc_duty(p, W, H, x, y, bw, be, bn, bs);
+  }
 }
 
 // setVBCs after advect (simulation.cpp:369) fused with project's divergence
@@ -709,6 +919,47 @@ __global__ void k_vbcs_divergence(const float *__restrict__ xf, const float *__r
                                   BCGrid gy) {
   vbcs_divergence_cell(blockIdx.x * blockDim.x + threadIdx.x + 1, blockIdx.y + 1, xf, yf, f, W, H,
                        ih, gx, gy);
+}
+
+// the same on wide rows
+__global__ void __launch_bounds__(64 * WIDE_WAVES)
+    k_vbcs_divergence_wide(const float *__restrict__ xf, const float *__restrict__ yf,
+                           float *__restrict__ f, int W, int H, float ih, BCGrid gx, BCGrid gy) {
+  const WideRow S(W, H);
+  const int Wx = W - 1, Hy = H - 1, y = S.y;
+  if (y == 0) return;
+  const bool north = y == Hy - 1;
+  float vx[2], vn[2], vs[2], fv[2];
+  S.loads([&](auto whole) {
+    constexpr bool K = decltype(whole)::value;
+    S.template load<K>(vx, xf, Wx, y);
+    S.template load<K>(vn, yf, W, y);
+    S.template load<K>(vs, yf, W, y - 1);
+  });
+  const float left = from_left(vx[1]);
+  if (S.inner) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) fv[c] = -ih * (vx[c] - (c ? vx[0] : left) + vn[c] - vs[c]);
+    S.store(f, W, fv, W - 2);
+    return;
+  }
+#pragma unroll
+  for (int c = 0; c < 2; c++) { // as vbcs_divergence_cell
+    const int x = S.x + c;
+    const bool east = x == Wx - 1;
+    const float xw = c ? vx[0] : left, ys = vs[c];
+    const float xe = (!east || gx.pe == BC_INFLOW) ? vx[c] : 0.0f;
+    const float yn = (!north || gy.pn == BC_INFLOW) ? vn[c] : 0.0f;
+    const float vx_w = (x == 1) ? bc_we(gx, gx.pw, xe, xw) : xw;
+    const float vx_e = east ? bc_we(gx, gx.pe, xw, xe) : xe;
+    const float vy_s = (y == 1) ? bc_sn(gy, gy.ps, yn, ys) : ys;
+    const float vy_n = north ? bc_sn(gy, gy.pn, ys, yn) : yn;
+    fv[c] = -ih * (vx_e - vx_w + vy_n - vy_s);
+    if (!S.owns(x, W - 2)) continue;
+    if (x <= Wx - 2) bc_duty(gx, x, y, xe, nullptr);
+    if (y <= Hy - 2) bc_duty(gy, x, y, yn, nullptr);
+  }
+  S.store(f, W, fv, W - 2);
 }
 
 // scalar bilinearSample (interpolators.hpp:11-27), clamp to [0, n-1.1]
@@ -970,26 +1221,49 @@ void launch_set_vbcs_vy(const VelView &v, const BCs &bc, hipStream_t s) {
 void launch_face_masks(const uint8_t *flag, uint16_t *fmask, int W, int H, hipStream_t s) {
   hipLaunchKernelGGL(k_face_masks, dim3(ceil_div(W, TPB), H), dim3(TPB), 0, s, flag, fmask, W, H);
 }
+// Whether a pass takes wide rows, and its grid.  One cell a lane is the faster
+// form while the fields stay in the 256 MB last-level cache, two cells a lane
+// where they come from memory, the sooner the more a pass is loads and stores
+// (us, one cell / two): divergence from 2.5M cells (2.1M 10.3 / 10.2, 3.4M
+// 14.2 / 12.0, 8.4M 28.9 / 22.0, 33.6M 125 / 87), correction from 5M (4.5M
+// 22.3 / 24.4, 6.0M 32.3 / 31.3, 8.4M 51 / 45, 33.6M 184 / 170), diffuse
+// beyond 9M (6.0M 27 / 30, 8.4M 39.6 / 40.8, 33.6M 184 / 131; one row a wave
+// instead of two: 146).
+enum WidePass { WIDE_FROM_DIVERGENCE = 2500000, WIDE_FROM_CORRECT = 5000000, WIDE_FROM_DIFFUSE = 9000000 };
+static bool wide_rows(int W, int H, WidePass from, int rows, dim3 *grid) {
+  const bool wide = (long)W * H >= from;
+  const unsigned band = 8 * WIDE_BAND;
+  *grid = wide ? dim3(ceil_div(W - 1, WIDE),
+                      ceil_div(ceil_div(H - 2, WIDE_WAVES * rows), band) * band)
+               : dim3(ceil_div(W - 2, TPB), H - 2);
+  return wide;
+}
 void launch_diffuse_both(const VelView &v, const uint16_t *fmask, float a, const BCs &bc,
                          hipStream_t s) {
   BCGrid gx{v.vxb, v.vxf, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyb, v.vyf, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
-  hipLaunchKernelGGL(k_diffuse_both, dim3(ceil_div(v.W - 2, TPB), v.H - 2), dim3(TPB), 0, s, v.vxf,
-                     v.vxb, v.vyf, v.vyb, fmask, v.W, v.H, a, gx, gy);
+  dim3 grid;
+  auto k = wide_rows(v.W, v.H, WIDE_FROM_DIFFUSE, WIDE_DIFFUSE, &grid) ? k_diffuse_wide
+                                                                       : k_diffuse_both;
+  hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vxb, v.vyf, v.vyb, fmask, v.W, v.H, a, gx,
+                     gy);
 }
 void launch_vbcs_divergence(const VelView &v, const BCs &bc, float *f, float ih, hipStream_t s) {
   BCGrid gx{v.vxf, v.vxb, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyf, v.vyb, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
-  hipLaunchKernelGGL(k_vbcs_divergence, dim3(ceil_div(v.W - 2, TPB), v.H - 2), dim3(TPB), 0, s,
-                     v.vxf, v.vyf, f, v.W, v.H, ih, gx, gy);
+  dim3 grid;
+  auto k = wide_rows(v.W, v.H, WIDE_FROM_DIVERGENCE, 1, &grid) ? k_vbcs_divergence_wide
+                                                               : k_vbcs_divergence;
+  hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vyf, f, v.W, v.H, ih, gx, gy);
 }
 void launch_correct_tail(const VelView &v, float *p, const uint16_t *fmask, float ih,
                          const BCs &bc, float *xcur, float *ycur, hipStream_t s) {
   BCGrid gx{v.vxf, v.vxb, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyf, v.vyb, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
-  hipLaunchKernelGGL(k_correct_tail, dim3(ceil_div(v.W - 2, TPB), v.H - 2), dim3(TPB), 0, s, v.vxf,
-                     v.vyf, p, fmask, v.W, v.H, ih, gx, gy, xcur, ycur, bc.west, bc.east, bc.north,
-                     bc.south);
+  dim3 grid;
+  auto k = wide_rows(v.W, v.H, WIDE_FROM_CORRECT, 1, &grid) ? k_correct_tail_wide : k_correct_tail;
+  hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vyf, p, fmask, v.W, v.H, ih, gx, gy, xcur,
+                     ycur, bc.west, bc.east, bc.north, bc.south);
 }
 void launch_set_pbc(float *p, int W, int H, const BCs &bc, hipStream_t s) {
   int n = W > H ? W : H;
