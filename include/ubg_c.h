@@ -217,9 +217,9 @@ UBG_API int ubg_mg_ir_device_ptrs(ubg_mg *mg, double **x, float **f);
  * problem of ubg_mg_ir_solve) on domains of uneven sizes, advanced together.
  * Every multigrid stage is one launch over a tile list spanning all domains
  * (sweeps, residual+restriction, prolongation+correction; the coarse levels
- * of each domain in one LDS workgroup), and a refinement step of all domains
- * (V-cycles, FP64 update, per-domain norm and convergence test) is replayed as
- * a captured hipGraph; a converged domain drops out on the device.  Each
+ * of each domain in one LDS workgroup), and the refinement steps of all
+ * domains (V-cycles, FP64 update, per-domain norm and convergence test) are
+ * enqueued two at a time; a converged domain drops out on the device.  Each
  * domain's result is bit-identical to ubg_mg_ir_solve on that domain alone.
  * Domains need W, H >= 16. */
 typedef struct ubg_batch ubg_batch;
@@ -244,7 +244,8 @@ UBG_API int ubg_batch_set_rhs(ubg_batch *b, int d, const float *rhs);
 /* float64 initial guess incl. the Dirichlet ring; NULL = 0 */
 UBG_API int ubg_batch_set_guess(ubg_batch *b, int d, const double *x);
 /* solve every domain to prm->tol (relative to its own initial residual);
- * UBG_E_NOT_CONVERGED if any domain stopped short (see ubg_batch_result) */
+ * UBG_E_NOT_CONVERGED if any domain stopped short (see ubg_batch_result);
+ * graph_replays (may be null): rounds of two steps */
 UBG_API int ubg_batch_solve(ubg_batch *b, const ubg_ir_params *prm, int *graph_replays);
 UBG_API int ubg_batch_result(ubg_batch *b, int d, ubg_ir_result *res);
 UBG_API int ubg_batch_get_solution(ubg_batch *b, int d, double *x);

@@ -66,7 +66,7 @@ class Batch:
         check(lib().ubg_batch_set_guess(self._h, d, x.ctypes.data_as(C.POINTER(C.c_double))))
 
     def solve(self, tol=1e-6, vcycles_per_iter=4, max_iter=200, raise_on_stall=True):
-        """Solve every domain; returns the number of two-step graph replays."""
+        """Solve every domain; returns the number of two-step rounds."""
         prm = L.IRParams(tol, vcycles_per_iter, max_iter)
         reps = C.c_int()
         rc = lib().ubg_batch_solve(self._h, C.byref(prm), C.byref(reps))

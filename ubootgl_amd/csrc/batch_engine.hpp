@@ -113,6 +113,24 @@ struct BShape {
 };
 int batch_shape(int W, int H, BShape *s);
 
+// Host tables on their way to the device: pinned staging and a device copy per
+// slot, the slots used in turn, so that neither side waits for the other.  A
+// slot's device copy belongs to the work queued between its put and the next;
+// it is written again once that work has passed.
+class UploadRing {
+public:
+  ~UploadRing();
+  int put(const void *data, size_t bytes, hipStream_t s, char **dev);
+
+private:
+  struct Slot {
+    char *host = nullptr, *dev = nullptr;
+    size_t cap = 0;
+    hipEvent_t used = nullptr; // recorded behind the slot's users
+  } slot_[4];
+  int cur_ = -1;
+};
+
 class BatchEngine {
 public:
   ~BatchEngine();
@@ -143,6 +161,9 @@ public:
   int domain_start(BDomain *d, double tol, int max_iter, double ref = 0.0,
                    hipStream_t s = nullptr);
   int domain_read_state(BDomain *d, DState *out, hipStream_t s = nullptr);
+  // the same for several domains at once, on the engine's stream
+  int start_all(const std::vector<BDomain *> &doms, double tol, int max_iter);
+  int read_states(const std::vector<BDomain *> &doms, std::vector<DState> &out);
   int domain_get_solution(BDomain *d, double *x_host, hipStream_t s = nullptr);
   // level-0 pressure and rhs of the plain V-cycles (projection solves); kind
   // is a hipMemcpyKind (host or device arrays); p == nullptr clears p
@@ -167,8 +188,6 @@ public:
   int enqueue_steps(int nsteps);
   // the first update (r0, no V-cycles) of every member, as if all were fresh
   int enqueue_first_update();
-  // eager steps, or one captured graph per index state, replayed
-  int run_steps_graph(int nsteps);
   // ncycles plain FP32 V-cycles (MG::solve, pressure_solver.cpp:250-257) of
   // every running member on its level-0 pressure and rhs; zg: level 0 takes
   // setZeroGradientBC after every sweep and after the correction (the
@@ -208,17 +227,17 @@ private:
   std::vector<BDomain *> run_, fresh_, all_;
   int lmax_ = 0;
   // device tables
-  BLev *d_lev_ = nullptr;
+  UploadRing tab_ring_, off_ring_, idx_ring_, st_ring_;
+  BLev *d_lev_ = nullptr; // in tab_ring_, as are d_dom_ and d_cargs_
   BDom *d_dom_ = nullptr;
   CoarseArgs *d_cargs_ = nullptr;
-  size_t tab_cap_ = 0;
+  size_t act_cap_ = 0;
   size_t coarse_lds_ = 0;
   bool coarse_big_ = false; // a member's first LDS level needs the larger variant
   // tile maps: per level sweep / rr / pc (running members), update (all):
   // prefix of tile counts over slots and tiles per row, in one int array
   std::vector<int> h_off_;
-  int *d_off_ = nullptr;
-  size_t off_cap_ = 0;
+  int *d_off_ = nullptr; // in off_ring_
   struct Span {
     size_t off = 0; // into the int array
     int n = 0;      // tiles
@@ -232,16 +251,11 @@ private:
   // levels run as the pre / post passes (smoothing counts that they take)
   bool tiled() const { return prm_.nu_pre <= kNuPass && prm_.nu_post <= kNuPass; }
   int launch_passes_only(int reps);
-  // stage index rows
-  uint8_t *d_idx_ = nullptr;
-  size_t idx_cap_ = 0;
-  uint8_t *h_idx_pinned_ = nullptr;
-  size_t h_idx_cap_ = 0;
   int *d_count_ = nullptr;
   int *count_host_ = nullptr;
   uint8_t *d_active_ = nullptr; // per slot, written with the count
   uint8_t *h_active_ = nullptr; // pinned copy
-  // graphs by index state (batched solves with a fixed member set)
+  // graphs by index state (projection batches with a fixed member set)
   struct Graph {
     hipGraphExec_t exec = nullptr;
     uint8_t *d_idx = nullptr;
