@@ -68,6 +68,16 @@ def test_level_passes_bit_exact(gpu, W, H, nu, kind, alpha, zg):
     mg.close()
 
 
+# more than 32 tiles per CU: the 12-wave shape of 6 rows, in one column of
+# tiles, in two whose second owns a few columns, and in three (whole tiles of
+# uniform rows in the middle)
+@pytest.mark.parametrize("W,H,kind", [(20, 164101, "noise"), (115, 82107, "noise"),
+                                      (300, 55013, "open")])
+@pytest.mark.parametrize("zg", [False, True])
+def test_largest_shape_bit_exact(gpu, W, H, kind, zg):
+    test_level_passes_bit_exact(gpu, W, H, 3, kind, 1.0, zg)
+
+
 # domains so elongated that the coarsest solved level is larger than the LDS
 # V-cycle's usual first level (4, 6 pairs of cells per thread), beside an
 # ordinary one and ones whose LDS levels have odd widths and one or two pairs

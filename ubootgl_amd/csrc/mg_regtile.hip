@@ -16,7 +16,7 @@ __device__ __forceinline__ void tile_origin(int ntx, int otx, int oty, int &X0, 
 }
 
 template <class T, bool ZP, bool ZG>
-__global__ void __launch_bounds__(T::TPB, 4)
+__global__ void __launch_bounds__(T::TPB, T::MINW)
     k_level_pre(const float *__restrict__ p, float *__restrict__ p_out,
                 const float *__restrict__ f, const uint8_t *__restrict__ m, int w, int h,
                 float hh, float alpha, float ihsq, float *__restrict__ fc,
@@ -29,7 +29,7 @@ __global__ void __launch_bounds__(T::TPB, 4)
 }
 
 template <class T, bool ZG>
-__global__ void __launch_bounds__(T::TPB, 4)
+__global__ void __launch_bounds__(T::TPB, T::MINW)
     k_level_post(const float *__restrict__ p, float *__restrict__ p_out,
                  const float *__restrict__ f, const uint8_t *__restrict__ m, int w, int h,
                  float hh, float alpha, const float *__restrict__ ec,
@@ -52,8 +52,16 @@ long tiles(const Level &L, PassShape shape, bool pre, int nu) {
   pass_tile(shape, pre, nu, &otx, &oty);
   return (long)((L.w + otx - 1) / otx) * ((L.h + oty - 1) / oty);
 }
-PassShape shape_of(const Level &L, bool pre, int nu) {
-  return pass_shape(tiles(L, PASS_TINY, pre, nu), tiles(L, PASS_SMALL, pre, nu));
+// fn(the level's RegTile).  Beyond the shapes of pass_shape: three sweeps on
+// more than 32 tiles per CU take 12 waves of 6 rows, whose halo is an even
+// smaller share (8192x4096 under the zero-gradient BC 143 + 131 us against 158
+// + 133 with 8 waves, without it 129 + 114 against 158 + 125; 4096x2048 41.0 +
+// 38.6 against 41.4 + 39.4, 2048x1024 18.5 + 18.4 against 17.4 + 17.3; with
+// two sweeps the post pass loses, 126 against 118 at 8192x4096).
+template <class Fn> void with_level(const Level &L, bool pre, int nu, Fn fn) {
+  const long small = tiles(L, PASS_SMALL, pre, nu);
+  if (nu == 3 && small > 32 * kPassCUs) fn(RegTile<3, 6, 12>{});
+  else with_pass(pass_shape(tiles(L, PASS_TINY, pre, nu), small), nu, fn);
 }
 
 void swap_p(Level &L) {
@@ -66,7 +74,7 @@ void swap_p(Level &L) {
 
 void launch_level_pre(Level &L, Level &C, int nu, float h, float alpha, bool zero_p, bool zg,
                       bool zero_coarse, hipStream_t s) {
-  with_pass(shape_of(L, true, nu), nu, [&](auto t) {
+  with_level(L, true, nu, [&](auto t) {
     using T = decltype(t);
     int otx, ntx, oty, nty;
     split(L.w, T::OTXP, otx, ntx);
@@ -82,7 +90,7 @@ void launch_level_pre(Level &L, Level &C, int nu, float h, float alpha, bool zer
 
 void launch_level_post(Level &L, const Level &C, int nu, float h, float alpha, bool zg,
                        hipStream_t s) {
-  with_pass(shape_of(L, false, nu), nu, [&](auto t) {
+  with_level(L, false, nu, [&](auto t) {
     using T = decltype(t);
     int otx, ntx, oty, nty;
     split(L.w, T::OTXQ, otx, ntx);
