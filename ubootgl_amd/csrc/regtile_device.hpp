@@ -94,10 +94,12 @@ __device__ __forceinline__ void stay_branch() { asm volatile(""); }
 template <int NU_, int RPW_, int WAVES_> struct RegTile {
   static constexpr int NU = NU_, CPL = 2, RPW = RPW_, WAVES = WAVES_;
   static constexpr int TPB = 64 * WAVES, COLS = 64 * CPL, ROWS = RPW * WAVES;
-  // waves per SIMD to compile for: of the largest shape two workgroups a CU
-  // need 6 (82 registers instead of 80 leave one: pre 189 instead of 129 us at
-  // 8192x4096 without the zero-gradient BC)
-  static constexpr int MINW = WAVES * RPW > 64 ? 6 : 4;
+  // waves per SIMD to compile the single-domain passes for: with 6 rows, three
+  // workgroups of 8 waves or two of 12 a CU need 6 (82 registers instead of 80
+  // leave one less: pre without the zero-gradient BC 39.9 instead of 34.5 us at
+  // 4096x2048, 189 instead of 129 with 12 waves at 8192x4096).  The batched
+  // passes spill under that bound (24.9 us instead of 22.9) and keep 4.
+  static constexpr int MINW = RPW >= 6 ? 6 : 4;
   static_assert(RPW % 2 == 0, "a register's colour does not depend on the wave");
   // pre: residuals on [X0-1, X0+otx-1] read p on [X0-2, X0+otx]; each sweep
   // widens that by 2
