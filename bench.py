@@ -8,7 +8,7 @@ on the 16x8 level, velocity correction, BCs, *_current copy) followed by one
 RK2 tracer step.  Inputs are resident in HBM before the timed region.
 
 Prints ONE JSON line (rank 0): value = timesteps/s; roofline of the dominant
-kernel (level-0 red/black smoother sweep, 13 algorithmic bytes per cell);
+kernel by time (advect, or one of the two level-0 multigrid passes);
 cpu_baseline = the CPU oracle (oracle/, OpenMP) on a bounded sample of the
 same workload on this host.
 """
@@ -35,8 +35,8 @@ ADVECT_BYTES_PER_CELL = 17  # vx, vy r 8 + flag 1 + vx, vy w 8
 # vector peak: 157.3 TFLOP/s / (64 lanes x 2 flops of an FMA)
 VALU_PEAK_GINST = 157.3e3 / 128
 KERNEL_NAMES = {"sweep": "level-0 rbgs sweep (red + black, one launch)",
-                "pre": "level-0 fused pass: rbgs sweep + residual + restriction",
-                "post": "level-0 fused pass: prolongation + correction + rbgs sweep",
+                "pre": "level-0 pass: 2 rbgs sweeps + residual + restriction",
+                "post": "level-0 pass: prolongation + correction + 2 rbgs sweeps",
                 "advect": "advect: RK2 backtrace + 3 Catmull-Rom samples per face (vx and vy)"}
 
 
@@ -57,7 +57,7 @@ def main():
                     help="timesteps per CPU-baseline run (3 runs, the median reported)")
     ap.add_argument("--no-graph", action="store_true")
     ap.add_argument("--no-hbm-sweep", action="store_true",
-                    help="skip the level-0 sweep timed on 8192x4096 (working set > 256 MB)")
+                    help="skip the stand-alone sweep timed on 4096x2048 and 8192x4096")
     ap.add_argument("--copies", type=int, default=0,
                     help="step: after the run, N saveCurrentVelocityFields stages (plain "
                          "33.5 MB device copies; counter calibration)")
@@ -133,14 +133,15 @@ def main():
     log(f"timed: {args.steps} steps in {(t2 - t1):.3f}s -> {steps_per_s:.1f} steps/s")
 
     # dominant kernels: HIP events on the simulation's stream around every
-    # level-0 launch of the three multigrid kernels (plain rbgs sweep; fused
-    # sweep+residual+restriction; fused prolongation+correction+sweep) over an
-    # instrumented pass of the same steps
+    # launch of advect and of the two level-0 multigrid passes (both
+    # pre-smoothing sweeps + residual + restriction; prolongation + correction +
+    # both post-smoothing sweeps) over an instrumented pass of the same steps
     from ubootgl_amd import _lib as LL
     ninstr = max(10, min(args.steps, 50))
-    timers = ((LL.TIMER_SMOOTH_L0, "sweep", SMOOTH_BYTES_PER_CELL, SMOOTH_BYTES_PER_CELL),
-              (LL.TIMER_L0_PRE, "pre", PRE_PASS_BYTES, SMOOTH_BYTES_PER_CELL + RR_BYTES_PER_CELL),
-              (LL.TIMER_L0_POST, "post", POST_PASS_BYTES, PC_BYTES_PER_CELL + SMOOTH_BYTES_PER_CELL),
+    timers = ((LL.TIMER_L0_PRE, "pre", PRE_PASS_BYTES,
+               2 * SMOOTH_BYTES_PER_CELL + RR_BYTES_PER_CELL),
+              (LL.TIMER_L0_POST, "post", POST_PASS_BYTES,
+               PC_BYTES_PER_CELL + 2 * SMOOTH_BYTES_PER_CELL),
               (LL.TIMER_ADVECT, "advect", ADVECT_BYTES_PER_CELL, ADVECT_BYTES_PER_CELL))
     for t, *_ in timers:
         sim.timer_enable(t, True)
@@ -188,20 +189,17 @@ def main():
                 "frac": round(rate / VALU_PEAK_GINST, 4),
                 "source": "instructions per launch from the same profile (SQ_INSTS_VALU), "
                           "divided by this run's launch time"}
-    sw = kern.get("sweep")
-    smoother = None if sw is None else {
-        "kernel": KERNEL_NAMES["sweep"], "achieved": round(sw["pass_GBps"], 1),
-        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(sw["pass_GBps"] / HBM_PEAK_GBS, 4),
-        "avg_launch_us": round(sw["avg_us"], 3),
-        "traffic": prof.get("sweep", {}).get("bytes_per_launch")}
-
     for _ in range(args.copies):
         sim.stage(LL.STAGE_SAVE_CURRENT, dt)
     sim.sync()
     vxg = sim.get("vx")
     finite = bool(np.isfinite(vxg).all())
     sim.close()
-    smoother_big = None if args.no_hbm_sweep else smoother_out_of_cache()
+    # the stand-alone sweep (the rbgs entry point; the step's sweeps run inside
+    # its level passes), in cache and out of it
+    smoother = smoother_big = None
+    if not args.no_hbm_sweep:
+        smoother, smoother_big = sweep_rate(4096, 2048), sweep_rate(8192, 4096)
 
     cpu = None
     if not args.no_cpu:
@@ -255,17 +253,16 @@ def main():
     print(json.dumps(out), flush=True)
 
 
-def smoother_out_of_cache(nsweeps=40):
-    """The level-0 red/black sweep on an 8192x4096 grid: p, p_alt and f
-    (134 MB each) plus the mask byte make a 436 MB working set, above the
-    256 MB Infinity Cache, so the achieved rate is HBM's.  Timed with the
-    dispatch-attached events over `nsweeps` back-to-back sweeps."""
+def sweep_rate(W, H, nsweeps=40):
+    """The red/black sweep alone on a W x H grid, timed with the
+    dispatch-attached events over `nsweeps` back-to-back sweeps.  At 8192x4096
+    p, p_alt and f (134 MB each) plus the mask byte make a 436 MB working set,
+    above the 256 MB Infinity Cache, so the achieved rate is HBM's."""
     import numpy as np
 
     import ubootgl_amd as U
     from ubootgl_amd import _lib as LL
 
-    W, H = 8192, 4096
     g = np.random.default_rng(5)
     flag = np.ones((H, W), np.float32)
     flag[0, :] = flag[-1, :] = flag[:, 0] = flag[:, -1] = 0
@@ -290,7 +287,7 @@ def smoother_out_of_cache(nsweeps=40):
     sim.close()
     avg = ms / max(n, 1)
     gbs = SMOOTH_BYTES_PER_CELL * W * H / (avg * 1e-3) / 1e9
-    log(f"sweep 8192x4096: {n} launches, avg {avg * 1e3:.2f} us -> {gbs:.0f} GB/s "
+    log(f"sweep {W}x{H}: {n} launches, avg {avg * 1e3:.2f} us -> {gbs:.0f} GB/s "
         f"({wall * 1e6 / nsweeps:.2f} us per sweep by wall clock)")
     return {"kernel": KERNEL_NAMES["sweep"], "grid": f"{W}x{H}",
             "working_set_MB": round(13 * W * H / 1e6, 1),  # p, p_alt, f + mask
@@ -378,7 +375,7 @@ def bench_batch(args):
     res = [bt.result(d) for d in range(len(probs))]
     batched = len(probs) * steps / el
     log(f"batched: {steps} x {len(probs)} solves in {el:.3f}s -> {batched:.1f} solves/s, "
-        f"{reps} graph replays, iterations {min(r['iterations'] for r in res)}.."
+        f"{reps} rounds of two steps, iterations {min(r['iterations'] for r in res)}.."
         f"{max(r['iterations'] for r in res)}")
     # sequential plain-GPU solves of the same problems
     mgs = []
