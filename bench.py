@@ -26,7 +26,7 @@ SMOOTH_BYTES_PER_CELL = 13  # one red+black sweep: p r/w 8 + f 4 + flag 1
 RR_BYTES_PER_CELL = 10      # residual + restriction (p 4, f 4, flag 1, coarse rhs 1)
 PC_BYTES_PER_CELL = 10.25   # prolongation + correction (coarse 1, coarse flag 0.25, flag 1, p r/w 8)
 # compulsory HBM bytes per cell of the two fused level-0 passes
-PRE_PASS_BYTES = 15.0       # p r 4 + f 4 + flag 1 + p w 4 + coarse rhs w 1 + coarse p w 1
+PRE_PASS_BYTES = 14.0       # p r 4 + f 4 + flag 1 + p w 4 + coarse rhs w 1
 POST_PASS_BYTES = 14.25     # p r 4 + f 4 + flag 1 + coarse p 1 + coarse flag 0.25 + p w 4
 STEP_BYTES_PER_CELL_22 = 278.6  # step at 2/2 smoothing, 2 V-cycles (algorithmic)
 TRACER_BYTES = 24  # xy r/w 16 + age r/w 8 per point

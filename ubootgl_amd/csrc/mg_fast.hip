@@ -1,6 +1,6 @@
 // mg_fast.hip -- fused multigrid kernels for gfx950.
 //
-// 1. k_rbgs_stream: one full red+black sweep of rbgs (pressure_solver.cpp:49-89,
+// 1. k_rbgs_pair: one full red+black sweep of rbgs (pressure_solver.cpp:49-89,
 //    two-pass semantics) in one launch.  Each wave streams down a strip of
 //    columns holding rows of p in registers; the red cells of row y+1 are
 //    updated before the black cells of row y, which is exactly the order the
@@ -16,7 +16,7 @@
 // 2. k_coarse_vcycle: the V-cycle of every level from `first` down to the
 //    coarsest solved level L-2 (pressure_solver.cpp:201-248), run by one
 //    workgroup entirely in LDS (p, f and mask of all those levels fit in
-//    160 KB once the level is <= ~128x64).  Replaces ~40 latency-bound
+//    160 KB once the level is <= ~128x64; it starts at 4096 cells).  Replaces ~40 latency-bound
 //    launches per V-cycle with one.
 #include "coarse_device.hpp"
 #include "stream_device.hpp"
