@@ -1,7 +1,7 @@
 """Coarse flags and neighbour masks (updateFields, pressure_solver.hpp:40-57)
 computed several levels a launch, against the oracle: every level's flags,
 and the masks through two V-cycles, bit-identical.  Sizes on both sides of a
-64-cell tile and its three coarsenings, of the one-workgroup tail (16384
+64-cell tile and its coarsenings, of the one-workgroup tail (16384
 cells), hierarchies of 2 to 10 levels and elongated ones; the
 allocation-free solve on top, with flag bytes other than 0 and 1, whose
 scratch holds the contents of the call before."""

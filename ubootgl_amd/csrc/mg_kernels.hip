@@ -77,29 +77,30 @@ __global__ void k_build_mask(const uint8_t *__restrict__ fl, uint8_t *__restrict
 // The flags of level l + 1 need those of level l, so a launch a level (and one
 // more for its mask, and a fill of the coarse fields) leaves a hierarchy's
 // set-up to launch latency: at 1025x1025 20 launches of 2 to 8 us.  Here a
-// workgroup takes a 64x64 tile of a level with the halo that three coarsenings
-// reach (7 cells before it, 4 behind), keeps the flags of all four levels in
+// workgroup takes a 64x64 tile of a level with the halo that four coarsenings
+// reach (15 cells before it, 8 behind), keeps the flags of its levels in
 // LDS and writes the tile's masks and coarse flags; a level of at most
 // kClassRest cells and all below it are one workgroup's, bound by its
-// passes' latency.  1025x1025: 8.3 + 14.9 us for two launches instead of 55 us
-// and 18 launch gaps; the allocation-free V-cycle on it 126 -> 96 us.  (A
-// tail from 32x32 cells costs one more launch of the first kind.)
+// passes' latency.  1025x1025: 8.6 + 9.6 us for two launches instead of 55 us
+// and 18 launch gaps; the allocation-free V-cycle on it 126 -> 91 us.  (With
+// three coarsenings a launch, and so a tail from 128x128 cells instead of
+// 64x64, 8.3 + 14.9.)
 //
 // Flags are bytes 0 / 1, so four cells' masks are one word: each neighbour's
 // bit and its count (bits 5..7) come from one multiply-add, and no byte of a
 // sum exceeds 159.
 constexpr int CLT = 64;           // cells of a tile
-constexpr int CLP0 = 80, CLH0 = CLT + 11; // first level's LDS rows (words of 4 cells from X0 - 8)
-constexpr int CLR1 = CLT / 2 + 5, CLR2 = CLT / 4 + 2;
+constexpr int CLP0 = 88, CLH0 = CLT + 23; // first level's LDS rows (words of 4 cells from X0 - 16)
+constexpr int CLR1 = CLT / 2 + 11, CLR2 = CLT / 4 + 5, CLR3 = CLT / 8 + 2;
 constexpr int kClassThreads = 1024, kClassRest = 16384;
 typedef uint32_t word_u __attribute__((aligned(1)));
 struct ClassStage {
   const uint8_t *src;     // flags of the first level
   uint8_t *copy;          // first level's flags as 0 / 1 (null: not written)
-  uint8_t *flag[4], *mask[3];
-  float *zero[4][3];      // fields of the coarse levels to clear (null: none)
-  int w[4], h[4];
-  int n;                  // levels below the first: 0 .. 3
+  uint8_t *flag[5], *mask[4];
+  float *zero[5][3];      // fields of the coarse levels to clear (null: none)
+  int w[5], h[5];
+  int n;                  // levels below the first: 0 .. 4
 };
 // masks of one cell or of four, from their flags and their neighbours'
 __device__ __forceinline__ unsigned mask_bytes(unsigned c, unsigned w, unsigned e, unsigned s,
@@ -118,15 +119,15 @@ __device__ __forceinline__ unsigned coarse_flag(const uint8_t *f, int pitch) {
 __global__ void __launch_bounds__(kClassThreads) k_classify(ClassStage a) {
   constexpr int PW = CLP0 / 4;
   __shared__ uint32_t f0_[CLH0 * PW + 2];
-  uint32_t *const f0 = f0_ + 1; // cell (x, y): byte x - X0 + 8 of row y - Y0 + 7
-  __shared__ uint8_t f1[CLR1 * CLR1], f2[CLR2 * CLR2];
+  uint32_t *const f0 = f0_ + 1; // cell (x, y): byte x - X0 + 16 of row y - Y0 + 15
+  __shared__ uint8_t f1[CLR1 * CLR1], f2[CLR2 * CLR2], f3[CLR3 * CLR3];
   const int X0 = blockIdx.x * CLT, Y0 = blockIdx.y * CLT, w0 = a.w[0], h0 = a.h[0];
   constexpr int NLD = (CLH0 * PW + kClassThreads - 1) / kClassThreads;
   uint32_t v0[NLD];
 #pragma unroll
   for (int k = 0; k < NLD; k++) {
     const int i = threadIdx.x + k * kClassThreads;
-    const int x = X0 - 8 + 4 * (i % PW), y = Y0 - 7 + i / PW;
+    const int x = X0 - 16 + 4 * (i % PW), y = Y0 - 15 + i / PW;
     v0[k] = 0u;
     if (y < 0 || y >= h0 || i >= CLH0 * PW) continue;
     const uint8_t *row = a.src + (size_t)y * w0;
@@ -148,7 +149,7 @@ __global__ void __launch_bounds__(kClassThreads) k_classify(ClassStage a) {
   { // the tile's masks, four cells a thread: 16 words x 64 rows
     static_assert(CLT / 4 * CLT == kClassThreads, "one word a thread");
     const int i = threadIdx.x % (CLT / 4), y = threadIdx.x / (CLT / 4), x = X0 + 4 * i;
-    const uint32_t *r = f0 + (y + 7) * PW + i + 2;
+    const uint32_t *r = f0 + (y + 15) * PW + i + 4;
     const uint32_t c = r[0], wst = (c << 8) | (r[-1] >> 24), e = (c >> 8) | (r[1] << 24);
     const uint32_t m = mask_bytes(c, wst, e, r[-PW], r[PW]);
     if (Y0 + y < h0) {
@@ -192,32 +193,36 @@ __global__ void __launch_bounds__(kClassThreads) k_classify(ClassStage a) {
   // level 1, two cells of a row from a word: the column sums of its three
   // rows, then each byte with its neighbours (at most 16).  The first cell of
   // word 0 lies outside the region.
-  if (threadIdx.x < CLR1 * (PW - 1)) {
-    const int i = threadIdx.x % (PW - 1), ry = threadIdx.x / (PW - 1);
-    const int y = (Y0 >> 1) - 3 + ry, x = (X0 - 8 + 4 * i) >> 1; // cells x, x + 1
-    const uint32_t *r = f0 + (2 * ry + 1) * PW + i;              // row 2 y
+  static_assert(CLR1 * PW <= kClassThreads, "one word a thread");
+  if (threadIdx.x < CLR1 * PW) {
+    const int i = threadIdx.x % PW, ry = threadIdx.x / PW;
+    const int y = (Y0 >> 1) - 7 + ry, x = (X0 - 16 + 4 * i) >> 1; // cells x, x + 1
+    const uint32_t *r = f0 + (2 * ry + 1) * PW + i;               // row 2 y
     auto column = [&](int d) { return r[d - PW] + 2u * r[d] + r[d + PW]; };
     const uint32_t c = column(0), l = (c << 8) | (column(-1) >> 24);
     const uint32_t t = l + 2u * c + (c >> 8); // bytes 0 and 2 are whole
-    put(1, x, y, (t & 0xffu) >= 4u, f1, CLR1, 3, CLT / 2);
-    put(1, x + 1, y, ((t >> 16) & 0xffu) >= 4u, f1, CLR1, 3, CLT / 2);
+    put(1, x, y, (t & 0xffu) >= 4u, f1, CLR1, 7, CLT / 2);
+    put(1, x + 1, y, ((t >> 16) & 0xffu) >= 4u, f1, CLR1, 7, CLT / 2);
   }
   __syncthreads();
-  masks(1, f1, CLR1, 3, CLT / 2);
+  masks(1, f1, CLR1, 7, CLT / 2);
+  // levels 2 .. 4: a region begins one cell into the double of the next
+  auto coarsen = [&](int k, const uint8_t *fine, int fr, uint8_t *out, int r, int lo, int t) {
+    if (threadIdx.x >= (unsigned)(r * r)) return;
+    const int rx = threadIdx.x % r, ry = threadIdx.x / r;
+    put(k, (X0 >> k) - lo + rx, (Y0 >> k) - lo + ry,
+        coarse_flag(fine + (2 * ry + 1) * fr + 2 * rx + 1, fr), out, r, lo, t);
+  };
   if (a.n < 2) return;
-  if (threadIdx.x < CLR2 * CLR2) {
-    const int rx = threadIdx.x % CLR2, ry = threadIdx.x / CLR2;
-    put(2, (X0 >> 2) - 1 + rx, (Y0 >> 2) - 1 + ry,
-        coarse_flag(f1 + (2 * ry + 1) * CLR1 + 2 * rx + 1, CLR1), f2, CLR2, 1, CLT / 4);
-  }
+  coarsen(2, f1, CLR1, f2, CLR2, 3, CLT / 4);
   __syncthreads();
-  masks(2, f2, CLR2, 1, CLT / 4);
+  masks(2, f2, CLR2, 3, CLT / 4);
   if (a.n < 3) return;
-  if (threadIdx.x < CLT / 8 * (CLT / 8)) {
-    const int rx = threadIdx.x % (CLT / 8), ry = threadIdx.x / (CLT / 8);
-    put(3, (X0 >> 3) + rx, (Y0 >> 3) + ry,
-        coarse_flag(f2 + (2 * ry + 1) * CLR2 + 2 * rx + 1, CLR2), nullptr, CLT / 8, 0, CLT / 8);
-  }
+  coarsen(3, f2, CLR2, f3, CLR3, 1, CLT / 8);
+  __syncthreads();
+  masks(3, f3, CLR3, 1, CLT / 8);
+  if (a.n < 4) return;
+  coarsen(4, f3, CLR3, nullptr, CLT / 16, 0, CLT / 16);
 }
 
 // the level of at most kClassRest cells and all below it: level k's flags in
@@ -486,17 +491,17 @@ void launch_classify(const Level *lv, int levels, const uint8_t *raw, bool zero,
   int l = 0;
   const uint8_t *src = raw ? raw : lv[0].flag;
   uint8_t *copy = raw ? lv[0].flag : nullptr;
-  for (; (size_t)lv[l].w * lv[l].h > kClassRest; l += 3) {
+  for (; (size_t)lv[l].w * lv[l].h > kClassRest; l += 4) {
     ClassStage a{};
     a.src = src;
     a.copy = copy;
-    a.n = levels - 1 - l < 3 ? levels - 1 - l : 3;
+    a.n = levels - 1 - l < 4 ? levels - 1 - l : 4;
     for (int k = 0; k <= a.n; k++) {
       const Level &L = lv[l + k];
       a.w[k] = L.w;
       a.h[k] = L.h;
       a.flag[k] = L.flag;
-      if (k < 3) a.mask[k] = L.mask;
+      if (k < 4) a.mask[k] = L.mask;
       if (zero && k > 0) {
         a.zero[k][0] = L.p;
         a.zero[k][1] = L.p_alt;
@@ -505,8 +510,8 @@ void launch_classify(const Level *lv, int levels, const uint8_t *raw, bool zero,
     }
     hipLaunchKernelGGL(k_classify, dim3(ceil_div(lv[l].w, CLT), ceil_div(lv[l].h, CLT)),
                        dim3(kClassThreads), 0, s, a);
-    if (l + 3 > levels - 1) return; // the last level's mask is written
-    src = lv[l + 3].flag;
+    if (l + 4 > levels - 1) return; // the last level's mask is written
+    src = lv[l + 4].flag;
     copy = nullptr;
   }
   ClassRest a{};
