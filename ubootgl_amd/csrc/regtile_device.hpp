@@ -29,7 +29,10 @@
 // four neighbours fluid (mask 0x9f) and alpha is 1, the update is
 // (((0 + W) + E + S) + N + (f h) h) / 4: no selects, and a product with 0.25,
 // which rounds as the division does.  One ballot per row decides it for all
-// sweeps; other rows take the constants from the LDS rule table.
+// sweeps; other rows take the constants from the LDS rule table.  A sum that
+// overflows gives NaN in both (the rule's quotient is corrected by v - 4 q =
+// inf - inf), so that a cell's value does not depend on the row and tile that
+// compute it.
 #pragma once
 
 #include "mg_device.hpp"
@@ -310,6 +313,7 @@ template <class T> struct TileRegs {
     v += north(i, c);
     v += F[i][c] * hh * hh;
     v *= 0.25f;                                // = v / 4
+    v = __builtin_fmaf(v, 0.0f, v);            // v, NaN for an infinite one
     return __builtin_fmaf(P[i][c], 0.0f, v);   // 1 v + 0 p
   }
   // colour phase: the cells with (c + i) & 1 == S
@@ -495,7 +499,7 @@ regtile_pre(char *smem, int X0, int Y0, int otx, int oty, const float *__restric
     v += t.east(i, c);
     v += t.south(i, c);
     v += t.north(i, c);
-    v = __builtin_fmaf(t.P[i][c], -4.0f, v); // v + (-4 p): the product is exact
+    v += -4.0f * t.P[i][c]; // the product apart: it may overflow where the sum would not
     v *= ihsq;
     return t.F[i][c] + v;
   };
