@@ -1,0 +1,158 @@
+// A batched solve whose allocations fail: the program takes the place of the
+// HIP runtime's memory, stream, event and launch calls (host memory, no
+// kernel runs), lets the k-th allocation of a call fail for every k, and
+// checks that the call says so and that the next call uploads what a call
+// after no failure uploads -- no table of an earlier member set or tuning is
+// taken for the present one.  Runs without a GPU.
+#include <ubg_c.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+namespace {
+constexpr int kOk = 0, kOutOfMemory = 2;
+int g_fail_at = 0, g_allocs = 0;      // the allocation to fail (0: none), those so far
+std::vector<size_t> g_uploads;        // sizes of the copies to the device
+struct Dim {
+  unsigned x, y, z;
+};
+Dim g_grid, g_block;
+size_t g_shared;
+void *g_stream;
+int take(void **p, size_t n) {
+  if (++g_allocs == g_fail_at) {
+    *p = nullptr;
+    return kOutOfMemory;
+  }
+  *p = std::calloc(1, n ? n : 1);
+  return kOk;
+}
+} // namespace
+
+extern "C" {
+int hipGetDeviceCount(int *n) { return *n = 1, kOk; }
+int hipGetDevice(int *d) { return *d = 0, kOk; }
+int hipGetLastError() { return kOk; }
+const char *hipGetErrorString(int e) { return e ? "out of memory" : "no error"; }
+int hipMalloc(void **p, size_t n) { return take(p, n); }
+int hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n); }
+int hipFree(void *p) { return std::free(p), kOk; }
+int hipHostFree(void *p) { return std::free(p), kOk; }
+int hipMemcpy(void *d, const void *s, size_t n, int) { return std::memcpy(d, s, n), kOk; }
+int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *) {
+  if (kind == 1) g_uploads.push_back(n);
+  return std::memcpy(d, s, n), kOk;
+}
+int hipMemset(void *d, int v, size_t n) { return std::memset(d, v, n), kOk; }
+int hipMemsetAsync(void *d, int v, size_t n, void *) { return std::memset(d, v, n), kOk; }
+int hipStreamCreateWithFlags(void **s, unsigned) { return *s = std::malloc(1), kOk; }
+int hipStreamSynchronize(void *) { return kOk; }
+int hipStreamDestroy(void *s) { return std::free(s), kOk; }
+int hipEventCreate(void **e) { return *e = std::malloc(1), kOk; }
+int hipEventCreateWithFlags(void **e, unsigned) { return *e = std::malloc(1), kOk; }
+int hipEventRecord(void *, void *) { return kOk; }
+int hipEventSynchronize(void *) { return kOk; }
+int hipEventElapsedTime(float *ms, void *, void *) { return *ms = 1.0f, kOk; }
+int hipEventDestroy(void *e) { return std::free(e), kOk; }
+int hipFuncSetAttribute(const void *, int, int) { return kOk; }
+int hipLaunchKernel(const void *, Dim, Dim, void **, size_t, void *) { return kOk; }
+int __hipPushCallConfiguration(Dim g, Dim b, size_t n, void *s) {
+  g_grid = g, g_block = b, g_shared = n, g_stream = s;
+  return kOk;
+}
+int __hipPopCallConfiguration(Dim *g, Dim *b, size_t *n, void **s) {
+  *g = g_grid, *b = g_block, *n = g_shared, *s = g_stream;
+  return kOk;
+}
+}
+
+namespace {
+int g_bad = 0;
+void expect(bool ok, const char *what, int k) {
+  if (ok) return;
+  std::printf("FAILED: %s (allocation %d fails; last error: %s)\n", what, k, ubg_last_error());
+  g_bad++;
+}
+
+ubg_batch *make(int n, int side) {
+  std::vector<int> w(n), h(n);
+  for (int d = 0; d < n; d++) {
+    w[d] = side + d;
+    h[d] = side;
+  }
+  ubg_batch *b = nullptr;
+  if (ubg_batch_create(n, w.data(), h.data(), nullptr, &b) != UBG_OK) std::exit(2);
+  for (int d = 0; d < n; d++) {
+    std::vector<float> one((size_t)w[d] * h[d], 1.0f);
+    if (ubg_batch_set_domain(b, d, one.data(), one.data(), 0.1f) != UBG_OK) std::exit(2);
+  }
+  return b;
+}
+
+// no kernel runs, so a call that reaches its end finds no converged domain
+bool reached_end(int rc) { return rc == UBG_E_NOT_CONVERGED; }
+
+// `call` on a batch that `before` has been applied to, its k-th allocation
+// failing for every k there is: the next solve's uploads are `want`, without
+// the tables and tile maps only where the failed call uploaded both (after the
+// states)
+template <class Before, class Call>
+void failing(const char *what, const std::vector<size_t> &want, Before before, Call call) {
+  for (int k = 1;; k++) {
+    ubg_batch *b = make(20, 40);
+    before(b);
+    g_allocs = 0;
+    g_fail_at = k;
+    g_uploads.clear();
+    const int rc = call(b);
+    const bool failed = g_allocs >= k, built = g_uploads.size() >= 3;
+    g_fail_at = 0;
+    if (failed) {
+      expect(rc == UBG_E_OOM, what, k);
+      g_uploads.clear();
+      expect(reached_end(ubg_batch_solve(b, nullptr, nullptr)), what, k);
+      const std::vector<size_t> rest = {want[0], want[3], want[4]};
+      expect(g_uploads == want || (built && g_uploads == rest), "uploads after a failure", k);
+    } else {
+      std::printf("%s: %d allocations\n", what, k - 1);
+    }
+    ubg_batch_destroy(b);
+    if (!failed) return;
+  }
+}
+} // namespace
+
+int main() {
+  // uploads of a solve that builds its tables: states, tables, tile maps,
+  // stage indices, states
+  ubg_batch *b = make(20, 40);
+  g_uploads.clear();
+  expect(reached_end(ubg_batch_solve(b, nullptr, nullptr)), "solve", 0);
+  const std::vector<size_t> want = g_uploads;
+  expect(want.size() == 5, "uploads of a first solve", 0);
+  ubg_batch_destroy(b);
+
+  auto nothing = [](ubg_batch *) {};
+  auto solve = [](ubg_batch *q) { return ubg_batch_solve(q, nullptr, nullptr); };
+  // one of the domains replaced, so that the tables of the former solve are
+  // another member set's
+  auto replaced = [&](ubg_batch *q) {
+    solve(q);
+    std::vector<float> one((size_t)40 * 40, 1.0f);
+    ubg_batch_set_domain(q, 0, one.data(), one.data(), 0.1f);
+  };
+  auto tune = [](ubg_batch *q) {
+    ubg_batch_tuning t{};
+    ubg_batch_get_tuning(q, &t);
+    t.pass_rows = 8;
+    return ubg_batch_set_tuning(q, &t);
+  };
+  failing("first solve", want, nothing, solve);
+  failing("solve after a domain was replaced", want, replaced, solve);
+  failing("a tuning after a solve", want, solve, tune);
+  if (g_bad) return 1;
+  std::printf("ALL OK\n");
+  return 0;
+}

@@ -813,9 +813,10 @@ int BatchEngine::set_members(const std::vector<BDomain *> &running,
   all_ = running;
   all_.insert(all_.end(), fresh.begin(), fresh.end());
   drop_graphs();
-  UBG_TRY(build_tables());
-  UBG_TRY(build_tiles());
-  return UBG_OK;
+  int rc = build_tables();
+  if (rc == UBG_OK) rc = build_tiles();
+  if (rc != UBG_OK) invalidate_members(); // the tables are an earlier set's
+  return rc;
 }
 
 int BatchEngine::build_tables() {
@@ -1271,10 +1272,12 @@ int BatchEngine::sync() {
   return UBG_OK;
 }
 
-void BatchEngine::set_tuning(const Tuning &t) {
+int BatchEngine::set_tuning(const Tuning &t) {
   tune_ = t;
   drop_graphs();
-  (void)build_tiles();
+  const int rc = build_tiles();
+  if (rc != UBG_OK) invalidate_members(); // the tile maps are the former tuning's
+  return rc;
 }
 
 // nu_pre sweeps of every member level, `reps` times (scratch buffers only:
@@ -1386,11 +1389,9 @@ int BatchEngine::autotune(double *best_ms) {
   (void)hipStreamSynchronize(stream_);
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
-  tune_ = rc == UBG_OK ? best : saved;
-  drop_graphs();
-  UBG_TRY(build_tiles());
+  const int rt = set_tuning(rc == UBG_OK ? best : saved);
   if (best_ms) *best_ms = best_t / 3.0;
-  return rc;
+  return rc != UBG_OK ? rc : rt;
 }
 
 } // namespace ubg
@@ -1904,8 +1905,7 @@ UBG_API int ubg_batch_set_tuning(ubg_batch *b, const ubg_batch_tuning *t) {
   const int rows = t->pass_rows;
   if (!pass_rows_ok(rows)) return fail(UBG_E_INVALID, "pass_rows must be 0, 8, 16 or 32");
   std::lock_guard<std::recursive_mutex> g(b->mu);
-  b->eng.set_tuning(ubg::Tuning{t->tile_w, t->tile_h, t->blocks, rows});
-  return UBG_OK;
+  return b->eng.set_tuning(ubg::Tuning{t->tile_w, t->tile_h, t->blocks, rows});
 }
 
 UBG_API int ubg_batch_get_tuning(ubg_batch *b, ubg_batch_tuning *t) {
@@ -1935,7 +1935,7 @@ UBG_API int ubg_batch_autotune(ubg_batch *b, const char *db_path, ubg_batch_tuni
       double ms;
       if (ls >> k >> tx >> ty >> bl >> rows >> ms && k == key && shape_ok(tx, ty) && bl >= 0 &&
           pass_rows_ok(rows)) {
-        b->eng.set_tuning(ubg::Tuning{tx, ty, bl, rows});
+        UBG_TRY(b->eng.set_tuning(ubg::Tuning{tx, ty, bl, rows}));
         if (out) *out = ubg_batch_tuning{tx, ty, bl, rows, ms};
         return UBG_OK;
       }

@@ -175,12 +175,13 @@ public:
   // and an accumulating update; `fresh` ones only their first update
   int set_members(const std::vector<BDomain *> &running, const std::vector<BDomain *> &fresh);
   // forget the member set (a member domain was replaced: a new domain may
-  // sit at the old one's address with other buffers), so the next
-  // set_members rebuilds the tables
+  // sit at the old one's address with other buffers; or its tables could not
+  // be built), so the next set_members rebuilds the tables
   void invalidate_members() {
     run_.clear();
     fresh_.clear();
     all_.clear();
+    d_lev_ = nullptr;
     drop_graphs();
   }
   // enqueue `nsteps` refinement steps of the members; the active-domain
@@ -199,7 +200,7 @@ public:
   size_t members() const { return all_.size(); }
   int sync();
 
-  void set_tuning(const Tuning &t);
+  int set_tuning(const Tuning &t);
   const Tuning &tuning() const { return tune_; }
   // time each compiled smoother tile shape and block count over the member
   // levels; keeps the fastest
