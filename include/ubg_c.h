@@ -497,9 +497,10 @@ UBG_API int ubg_sim_sync(ubg_sim *sim);
 
 /* ---- measurement ---------------------------------------------------------- */
 /* Kernel timing with HIP events attached to every dispatch of one kernel
- * class while enabled: level-0 stand-alone smoother passes, the level-0
- * fused pre-smoothing + residual + restriction pass, the level-0 fused
- * prolongation + correction + post-smoothing pass, and advect. */
+ * class while enabled: every level-0 launch that smooths (stand-alone sweeps
+ * and the two passes below, where they have sweeps), the level-0
+ * pre-smoothing + residual + restriction pass, the level-0 prolongation +
+ * correction + post-smoothing pass, and advect. */
 enum { UBG_TIMER_SMOOTH_L0 = 0, UBG_TIMER_L0_PRE, UBG_TIMER_L0_POST, UBG_TIMER_ADVECT,
        UBG_TIMER_COUNT };
 UBG_API int ubg_sim_timer_enable(ubg_sim *sim, int timer, int on);

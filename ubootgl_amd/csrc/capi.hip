@@ -1290,9 +1290,9 @@ UBG_API int ubg_sim_timer_enable(ubg_sim *s, int timer, int on) {
   std::lock_guard<std::recursive_mutex> g(s->mu_);
   s->enter();
   UBG_HIP(hipStreamSynchronize(s->stream));
+  for (Timer &x : s->timers) UBG_TRY(x.collect()); // a pair may serve two timers
   Timer &t = s->timers[timer];
   t.on = on != 0;
-  t.used = 0;
   t.total_ms = 0.0;
   t.launches = 0;
   return UBG_OK;
@@ -1303,14 +1303,8 @@ UBG_API int ubg_sim_timer_read(ubg_sim *s, int timer, double *total_ms, long *la
   std::lock_guard<std::recursive_mutex> g(s->mu_);
   s->enter();
   UBG_HIP(hipStreamSynchronize(s->stream));
-  Timer &t = s->timers[timer];
-  for (size_t i = 0; i + 1 < t.used; i += 2) {
-    float ms = 0.0f;
-    UBG_HIP(hipEventElapsedTime(&ms, t.ev[i], t.ev[i + 1]));
-    t.total_ms += ms;
-    t.launches++;
-  }
-  t.used = 0;
+  for (Timer &x : s->timers) UBG_TRY(x.collect());
+  const Timer &t = s->timers[timer];
   if (total_ms) *total_ms = t.total_ms;
   if (launches) *launches = t.launches;
   return UBG_OK;

@@ -101,26 +101,50 @@ inline int validate_flag(const float *flag, size_t n, std::vector<uint8_t> &out)
 struct Timer {
   bool on = false;
   std::vector<hipEvent_t> ev; // pairs
+  std::vector<Timer *> also;  // by pair: the timer that counts its launch as well (or null)
   size_t used = 0;
   double total_ms = 0.0;
   long launches = 0;
+  // the pairs' times, once their launches have ended
+  int collect() {
+    for (size_t i = 0; i + 1 < used; i += 2) {
+      float ms = 0.0f;
+      UBG_HIP(hipEventElapsedTime(&ms, ev[i], ev[i + 1]));
+      for (Timer *t : {this, also[i / 2]})
+        if (t) {
+          t->total_ms += ms;
+          t->launches++;
+        }
+    }
+    used = 0;
+    return UBG_OK;
+  }
 };
 
-// run `fn` (one kernel launch through launch_k) with the timer's next event
-// pair attached to its dispatch, when the timer is given and enabled
-template <typename Fn> void with_timer(Timer *t, Fn fn) {
-  const bool on = t && t->on;
-  if (on) {
+// run `fn` (one kernel launch through launch_k) with a timer's next event pair
+// attached to its dispatch, when a timer is given and enabled: t, and `also`
+// where the launch is of its class too (one pair serves both)
+template <typename Fn> void with_timer(Timer *t, Fn fn, Timer *also = nullptr) {
+  if (also && !also->on) also = nullptr;
+  if (!t || !t->on) {
+    t = also;
+    also = nullptr;
+  }
+  if (t) {
     if (t->used + 2 > t->ev.size()) {
       size_t n = t->ev.size();
       t->ev.resize(n + 512);
       for (size_t i = n; i < t->ev.size(); i++) (void)hipEventCreate(&t->ev[i]);
+      t->also.resize(t->ev.size() / 2);
     }
     g_launch_ev = LaunchEvents{t->ev[t->used], t->ev[t->used + 1]};
   }
   fn();
-  if (on) {
-    if (!g_launch_ev.start) t->used += 2; // the launch took the pair
+  if (t) {
+    if (!g_launch_ev.start) { // the launch took the pair
+      t->also[t->used / 2] = also;
+      t->used += 2;
+    }
     g_launch_ev = LaunchEvents{};
   }
 }
@@ -196,17 +220,19 @@ struct ubg_mg {
   std::recursive_mutex mu;
 
   // run `fn` (one kernel launch) with timer `id`'s next event pair attached
-  // to its dispatch when the timer is enabled and the work is on level 0
-  template <typename Fn> void timed(int id, int l, Fn fn) {
-    Timer *t = timers ? &timers[id] : nullptr;
-    with_timer(t && l == 0 ? t : nullptr, fn);
+  // to its dispatch when the timer is enabled and the work is on level 0; a
+  // launch with smoothing sweeps counts for UBG_TIMER_SMOOTH_L0 too
+  template <typename Fn> void timed(int id, int l, bool smooths, Fn fn) {
+    const bool t = timers && l == 0;
+    with_timer(t ? &timers[id] : nullptr, fn,
+               t && smooths && id != UBG_TIMER_SMOOTH_L0 ? &timers[UBG_TIMER_SMOOTH_L0] : nullptr);
   }
 
   // n sweeps at level l, one launch each
   void sweeps(int l, int n, float h, bool zg) {
     Level &L = lv[l];
     for (int i = 0; i < n; i++)
-      timed(UBG_TIMER_SMOOTH_L0, l, [&] { launch_rbgs_fused(L, h, prm.alpha, zg, stream); });
+      timed(UBG_TIMER_SMOOTH_L0, l, true, [&] { launch_rbgs_fused(L, h, prm.alpha, zg, stream); });
   }
 
   // Whether solve_level(l) (l > 0: zero initial guess, no ZG) reads its p
@@ -239,12 +265,12 @@ struct ubg_mg {
     Level &L = lv[l], &C = lv[l + 1];
     const int pre = std::min(prm.nu_pre, kNuPass), post = std::min(prm.nu_post, kNuPass);
     sweeps(l, prm.nu_pre - pre, h, z);
-    timed(UBG_TIMER_L0_PRE, l, [&] {
+    timed(UBG_TIMER_L0_PRE, l, pre > 0, [&] {
       launch_level_pre(L, C, pre, h, prm.alpha, l > 0 && prm.nu_pre <= kNuPass, z,
                        reads_zero_p(l + 1), stream);
     });
     solve_level(l + 1, h * (L.w - 1.0f) / (C.w - 1.0f), false); // pressure_solver.cpp:229
-    timed(UBG_TIMER_L0_POST, l,
+    timed(UBG_TIMER_L0_POST, l, post > 0,
           [&] { launch_level_post(L, C, post, h, prm.alpha, z, stream); });
     sweeps(l, prm.nu_post - post, h, z);
   }
