@@ -1436,8 +1436,13 @@ int batch_check(ubg_batch *b, int d) {
   return UBG_OK;
 }
 
+// The kernels that a line of a tuning file was timed with: counted up when its
+// numbers come to name other ones (2: pass_rows names shapes of register
+// tiles, before that rows of LDS tiles), so that an older line is timed anew.
+constexpr uint64_t kTuningKernels = 2;
 std::string batch_key(const ubg_batch *b, const ubg_params &p, int k) {
-  // FNV-1a over the sizes and the smoothing counts
+  // FNV-1a over the sizes, the smoothing counts, alpha (off 1 no row takes the
+  // uniform update) and the kernels
   uint64_t hsh = 1469598103934665603ull;
   auto mix = [&](uint64_t v) {
     for (int i = 0; i < 8; i++) {
@@ -1453,6 +1458,10 @@ std::string batch_key(const ubg_batch *b, const ubg_params &p, int k) {
   mix((uint64_t)p.nu_post);
   mix((uint64_t)p.nu_coarse);
   mix((uint64_t)k);
+  uint32_t alpha;
+  std::memcpy(&alpha, &p.alpha, sizeof alpha);
+  mix(alpha);
+  mix(kTuningKernels);
   char buf[40];
   std::snprintf(buf, sizeof(buf), "%016llx", (unsigned long long)hsh);
   return buf;
