@@ -3,9 +3,12 @@
 // kernel runs), lets the k-th allocation of a call fail for every k, and
 // checks that the call says so and that the next call uploads what a call
 // after no failure uploads -- no table of an earlier member set or tuning is
-// taken for the present one.  Runs without a GPU.
+// taken for the present one.  A handle allocates what it needs when it is
+// made: solves, tunings and a server's ordinary bursts allocate and free
+// nothing.  Runs without a GPU.
 #include <ubg_c.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -13,7 +16,8 @@
 
 namespace {
 constexpr int kOk = 0, kOutOfMemory = 2;
-int g_fail_at = 0, g_allocs = 0;      // the allocation to fail (0: none), those so far
+// the allocation to fail (0: none), allocations and releases so far
+std::atomic<int> g_fail_at{0}, g_allocs{0}, g_frees{0};
 std::vector<size_t> g_uploads;        // sizes of the copies to the device
 struct Dim {
   unsigned x, y, z;
@@ -38,8 +42,8 @@ int hipGetLastError() { return kOk; }
 const char *hipGetErrorString(int e) { return e ? "out of memory" : "no error"; }
 int hipMalloc(void **p, size_t n) { return take(p, n); }
 int hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n); }
-int hipFree(void *p) { return std::free(p), kOk; }
-int hipHostFree(void *p) { return std::free(p), kOk; }
+int hipFree(void *p) { return g_frees++, std::free(p), kOk; }
+int hipHostFree(void *p) { return g_frees++, std::free(p), kOk; }
 int hipMemcpy(void *d, const void *s, size_t n, int) { return std::memcpy(d, s, n), kOk; }
 int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *) {
   if (kind == 1) g_uploads.push_back(n);
@@ -152,6 +156,44 @@ int main() {
   failing("first solve", want, nothing, solve);
   failing("solve after a domain was replaced", want, replaced, solve);
   failing("a tuning after a solve", want, solve, tune);
+
+  // 60 domains, two solves and a tuning
+  b = make(60, 20);
+  g_allocs = g_frees = 0;
+  solve(b);
+  tune(b);
+  solve(b);
+  expect(g_allocs == 0 && g_frees == 0, "allocations of solves", 0);
+  ubg_batch_destroy(b);
+  expect(g_frees <= 3, "releases of a batch", 0);
+
+  // bursts of requests: two that a new server has tables for, larger ones, one
+  // of them with an allocation that fails (its requests may fail, the next
+  // ones do not)
+  ubg_server_params sp;
+  ubg_server_params_default(&sp);
+  sp.hbm_budget = (size_t)64 << 20;
+  ubg_server *srv = nullptr;
+  if (ubg_server_create(&sp, nullptr, &srv) != UBG_OK) return 2;
+  std::vector<float> one(24 * 20, 1.0f);
+  int geom = 0;
+  if (ubg_server_add_geometry(srv, 24, 20, one.data(), 0.1f, &geom) != UBG_OK) return 2;
+  g_frees = 0;
+  for (int n : {4, 60, 200, 500, 501}) {
+    const float *rhs[2] = {one.data(), one.data()};
+    const double fnorm[2] = {1.0, 1.0};
+    std::vector<uint64_t> id(n);
+    g_allocs = 0;
+    g_fail_at = n == 500 ? 1 : 0;
+    for (auto &i : id)
+      if (ubg_server_submit(srv, geom, 2, rhs, fnorm, nullptr, &i) != UBG_OK) return 2;
+    for (auto &i : id)
+      expect(ubg_server_wait(srv, i, -1.0, nullptr) == UBG_OK || n == 500, "request", n);
+    if (n <= 60) expect(g_allocs == 0, "allocations of a burst", n);
+    expect(g_frees == 0, "releases in a burst", n);
+    std::printf("burst of %d: %d allocations\n", n, (int)g_allocs);
+  }
+  ubg_server_destroy(srv);
   if (g_bad) return 1;
   std::printf("ALL OK\n");
   return 0;

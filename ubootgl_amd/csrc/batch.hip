@@ -515,29 +515,61 @@ int batch_shape(int W, int H, BShape *s) {
   return UBG_OK;
 }
 
-UploadRing::~UploadRing() {
-  for (Slot &q : slot_) {
-    if (q.host) (void)hipHostFree(q.host);
-    if (q.dev) (void)hipFree(q.dev);
-    if (q.used) (void)hipEventDestroy(q.used);
+Staging::~Staging() {
+  for (Block &b : blocks_) {
+    (void)hipHostFree(b.host);
+    (void)hipFree(b.dev);
   }
 }
 
-int UploadRing::put(const void *data, size_t bytes, hipStream_t s, char **dev) {
+int Staging::reserve(size_t bytes) {
+  if (!blocks_.empty() && blocks_.back().cap - blocks_.back().used >= bytes) return UBG_OK;
+  Block b;
+  for (const Block &q : blocks_) b.cap += q.cap;
+  b.cap = std::max(b.cap, al(bytes));
+  UBG_HIP(hipHostMalloc((void **)&b.host, b.cap, hipHostMallocDefault));
+  const hipError_t e = hipMalloc((void **)&b.dev, b.cap);
+  if (e != hipSuccess) {
+    (void)hipHostFree(b.host);
+    UBG_HIP(e);
+  }
+  blocks_.push_back(b);
+  return UBG_OK;
+}
+
+int Staging::carve(size_t bytes, char **host, char **dev) {
+  bytes = al(bytes);
+  UBG_TRY(reserve(bytes));
+  Block &b = blocks_.back();
+  *host = b.host + b.used;
+  *dev = b.dev + b.used;
+  b.used += bytes;
+  return UBG_OK;
+}
+
+UploadRing::~UploadRing() {
+  for (Slot &q : slot_)
+    if (q.used) (void)hipEventDestroy(q.used);
+}
+
+int UploadRing::reserve(Staging &st, size_t bytes) {
+  for (Slot &q : slot_) {
+    UBG_HIP(hipEventCreateWithFlags(&q.used, hipEventDisableTiming));
+    UBG_TRY(st.carve(bytes, &q.host, &q.dev));
+    q.cap = al(bytes);
+  }
+  return UBG_OK;
+}
+
+int UploadRing::put(Staging &st, const void *data, size_t bytes, hipStream_t s, char **dev) {
   if (cur_ >= 0) UBG_HIP(hipEventRecord(slot_[cur_].used, s));
-  cur_ = (cur_ + 1) % 4;
+  cur_ = (cur_ + 1) % SLOTS;
   Slot &q = slot_[cur_];
-  if (!q.used) UBG_HIP(hipEventCreateWithFlags(&q.used, hipEventDisableTiming));
   UBG_HIP(hipEventSynchronize(q.used)); // at once unless recorded and not passed
-  if (bytes > q.cap || !q.dev) {
-    if (q.host) (void)hipHostFree(q.host);
-    if (q.dev) (void)hipFree(q.dev);
-    q.host = q.dev = nullptr;
-    q.cap = 0;
-    const size_t cap = bytes + bytes / 2 + 256;
-    UBG_HIP(hipHostMalloc((void **)&q.host, cap, hipHostMallocDefault));
-    UBG_HIP(hipMalloc((void **)&q.dev, cap));
-    q.cap = cap;
+  if (bytes > q.cap) {
+    const size_t cap = 2 * bytes;
+    UBG_TRY(st.carve(cap, &q.host, &q.dev));
+    q.cap = al(cap);
   }
   *dev = q.dev;
   if (!bytes) return UBG_OK;
@@ -546,20 +578,36 @@ int UploadRing::put(const void *data, size_t bytes, hipStream_t s, char **dev) {
   return UBG_OK;
 }
 
-BatchEngine::~BatchEngine() {
-  drop_graphs();
-  if (d_count_) (void)hipFree(d_count_);
-  if (d_active_) (void)hipFree(d_active_);
-  if (h_active_) (void)hipHostFree(h_active_);
-  if (count_host_) (void)hipHostFree(count_host_);
+// sizes of the uploads for n member domains
+static size_t tables_bytes(size_t n) {
+  return al(n * BMAXL * sizeof(BLev)) + al(n * sizeof(BDom)) + n * sizeof(CoarseArgs);
 }
+static size_t states_bytes(size_t n) { return al(n * sizeof(DState *)) + n * sizeof(DState); }
 
-int BatchEngine::init(hipStream_t s, const ubg_params &prm, int vcycles_per_step) {
+BatchEngine::~BatchEngine() { drop_graphs(); }
+
+int BatchEngine::init(hipStream_t s, const ubg_params &prm, int vcycles_per_step, int members) {
   stream_ = s;
   prm_ = prm;
   k_ = vcycles_per_step;
-  UBG_HIP(hipMalloc((void **)&d_count_, sizeof(int)));
-  UBG_HIP(hipHostMalloc((void **)&count_host_, sizeof(int), hipHostMallocDefault));
+  // tile maps: sweep, residual and prolongation stages, the two passes of a
+  // level, the update; index rows: two steps of domains of eight levels, to 1 MB
+  const size_t n = (size_t)members, maps = (tiled() ? 5 : 3) * BMAXL + 1;
+  const size_t stages = tiled() ? 2 * 8 + 1 : 8 * ((size_t)prm_.nu_pre + prm_.nu_post + 2) + 1;
+  const size_t tab = tables_bytes(n), off = maps * (3 * n + 1) * sizeof(int),
+               idx = std::min(2 * (k_ * stages + 2) * 2 * n, size_t(1) << 20),
+               st = states_bytes(n);
+  UBG_TRY(staging_.reserve(UploadRing::SLOTS * (al(tab) + al(off) + al(idx) + al(st)) + al(n) +
+                           al(sizeof(int))));
+  UBG_TRY(tab_ring_.reserve(staging_, tab));
+  UBG_TRY(off_ring_.reserve(staging_, off));
+  UBG_TRY(idx_ring_.reserve(staging_, idx));
+  UBG_TRY(st_ring_.reserve(staging_, st));
+  UBG_TRY(reserve_active(n));
+  char *host, *dev;
+  UBG_TRY(staging_.carve(sizeof(int), &host, &dev));
+  count_host_ = (int *)host;
+  d_count_ = (int *)dev;
   *count_host_ = 0;
   static const bool attr_set = [] { // more than 64 KiB of LDS
     for (auto k : {kb_coarse<false>, kb_coarse<true>})
@@ -735,14 +783,14 @@ int BatchEngine::domain_read_state(BDomain *d, DState *out, hipStream_t s) {
 int BatchEngine::start_all(const std::vector<BDomain *> &doms, double tol, int max_iter) {
   const size_t n = doms.size(), ptr_bytes = al(n * sizeof(DState *));
   if (!n) return UBG_OK;
-  std::vector<char> blob(ptr_bytes + n * sizeof(DState));
+  std::vector<char> blob(states_bytes(n));
   for (size_t i = 0; i < n; i++) {
     ((DState **)blob.data())[i] = doms[i]->st;
     DState &st = ((DState *)(blob.data() + ptr_bytes))[i];
     st = start_state(tol, max_iter, 0.0, k_, doms[i]->xcur);
   }
   char *dev = nullptr;
-  UBG_TRY(st_ring_.put(blob.data(), blob.size(), stream_, &dev));
+  UBG_TRY(st_ring_.put(staging_, blob.data(), blob.size(), stream_, &dev));
   hipLaunchKernelGGL(kb_put_states, dim3((unsigned)n), dim3(64), 0, stream_, (DState *const *)dev,
                      (const DState *)(dev + ptr_bytes));
   return check_launch();
@@ -752,10 +800,10 @@ int BatchEngine::read_states(const std::vector<BDomain *> &doms, std::vector<DSt
   const size_t n = doms.size(), ptr_bytes = al(n * sizeof(DState *));
   out.resize(n);
   if (!n) return UBG_OK;
-  std::vector<char> blob(ptr_bytes + n * sizeof(DState));
+  std::vector<char> blob(states_bytes(n));
   for (size_t i = 0; i < n; i++) ((DState **)blob.data())[i] = doms[i]->st;
   char *dev = nullptr;
-  UBG_TRY(st_ring_.put(blob.data(), blob.size(), stream_, &dev));
+  UBG_TRY(st_ring_.put(staging_, blob.data(), blob.size(), stream_, &dev));
   hipLaunchKernelGGL(kb_get_states, dim3((unsigned)n), dim3(64), 0, stream_, (DState *const *)dev,
                      (DState *)(dev + ptr_bytes));
   UBG_TRY(check_launch());
@@ -819,22 +867,21 @@ int BatchEngine::set_members(const std::vector<BDomain *> &running,
   return rc;
 }
 
+int BatchEngine::reserve_active(size_t n) {
+  char *host, *dev;
+  UBG_TRY(staging_.carve(n, &host, &dev));
+  h_active_ = (uint8_t *)host;
+  d_active_ = (uint8_t *)dev;
+  std::memset(h_active_, 0, n);
+  act_cap_ = n;
+  return UBG_OK;
+}
+
 int BatchEngine::build_tables() {
   const size_t n = all_.size();
-  if (n > act_cap_) {
-    if (d_active_) (void)hipFree(d_active_);
-    if (h_active_) (void)hipHostFree(h_active_);
-    d_active_ = nullptr;
-    h_active_ = nullptr;
-    act_cap_ = 0;
-    size_t cap = std::max<size_t>(n, 16);
-    UBG_HIP(hipMalloc((void **)&d_active_, cap));
-    UBG_HIP(hipHostMalloc((void **)&h_active_, cap, hipHostMallocDefault));
-    std::memset(h_active_, 0, cap);
-    act_cap_ = cap;
-  }
+  if (n > act_cap_) UBG_TRY(reserve_active(2 * n));
   const size_t lev_bytes = al(n * BMAXL * sizeof(BLev)), dom_bytes = al(n * sizeof(BDom));
-  std::vector<char> blob(lev_bytes + dom_bytes + n * sizeof(CoarseArgs));
+  std::vector<char> blob(tables_bytes(n));
   BLev *lev = (BLev *)blob.data();
   BDom *dom = (BDom *)(blob.data() + lev_bytes);
   CoarseArgs *ca = (CoarseArgs *)(blob.data() + lev_bytes + dom_bytes);
@@ -891,7 +938,7 @@ int BatchEngine::build_tables() {
   }
   if (n) {
     char *dev = nullptr;
-    UBG_TRY(tab_ring_.put(blob.data(), blob.size(), stream_, &dev));
+    UBG_TRY(tab_ring_.put(staging_, blob.data(), blob.size(), stream_, &dev));
     d_lev_ = (BLev *)dev;
     d_dom_ = (BDom *)(dev + lev_bytes);
     d_cargs_ = (CoarseArgs *)(dev + lev_bytes + dom_bytes);
@@ -982,7 +1029,7 @@ int BatchEngine::build_tiles() {
     nx = all_[s]->gx;
     ny = all_[s]->gy;
   });
-  return off_ring_.put(h_off_.data(), h_off_.size() * sizeof(int), stream_, (char **)&d_off_);
+  return off_ring_.put(staging_, h_off_.data(), h_off_.size() * sizeof(int), stream_, (char **)&d_off_);
 }
 
 enum { ST_SWEEP, ST_RR, ST_PC, ST_COARSE, ST_UPDATE, ST_NORM, ST_TPRE, ST_TPOST };
@@ -1165,7 +1212,7 @@ int BatchEngine::launch_stages(const std::vector<StageRec> &st, const uint8_t *d
 }
 
 int BatchEngine::upload_idx(const std::vector<uint8_t> &idx, uint8_t **d_idx) {
-  return idx_ring_.put(idx.data(), idx.size(), stream_, (char **)d_idx);
+  return idx_ring_.put(staging_, idx.data(), idx.size(), stream_, (char **)d_idx);
 }
 
 int BatchEngine::enqueue_steps(int nsteps) {
@@ -1508,7 +1555,7 @@ UBG_API int ubg_batch_create(int n, const int *widths, const int *heights, const
   b->ready.assign(n, false);
   b->doms.assign(n, nullptr);
   int rc = b->arena.init(bytes + 4096);
-  if (rc == UBG_OK) rc = b->eng.init(b->stream, P, 4);
+  if (rc == UBG_OK) rc = b->eng.init(b->stream, P, 4, n);
   if (rc != UBG_OK) {
     ubg_batch_destroy(b);
     return rc;

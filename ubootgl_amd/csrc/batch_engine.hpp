@@ -113,28 +113,55 @@ struct BShape {
 };
 int batch_shape(int W, int H, BShape *s);
 
-// Host tables on their way to the device: pinned staging and a device copy per
-// slot, the slots used in turn, so that neither side waits for the other.  A
+// An engine's small memory: pinned host blocks with device blocks of the same
+// sizes, carved in pairs and kept until the engine ends.  One block made with
+// the engine holds what its members need; where they outgrow it, another at
+// least as large as those before it is added.  (A pair of allocations costs 175
+// us and its release as much, so sixteen of them, made by the first solves,
+// took a new server's first burst of four 32x32 requests from 1.7 to 2.4 ms and
+// the destruction of a batch of eight from 0.1 to 1.2 ms.)
+class Staging {
+public:
+  ~Staging();
+  int reserve(size_t bytes); // the next `bytes` come from one block
+  int carve(size_t bytes, char **host, char **dev);
+
+private:
+  struct Block {
+    char *host = nullptr, *dev = nullptr;
+    size_t cap = 0, used = 0;
+  };
+  std::vector<Block> blocks_;
+};
+
+// Host tables on their way to the device: two slots, used in turn, so that a
+// table is prepared while the work that reads the one before it runs.  A
 // slot's device copy belongs to the work queued between its put and the next;
-// it is written again once that work has passed.
+// it is written again once that work has passed.  (Solves and server turns end
+// with a synchronisation, so the slots' events have passed when they are waited
+// for.)
 class UploadRing {
 public:
+  static constexpr int SLOTS = 2;
   ~UploadRing();
-  int put(const void *data, size_t bytes, hipStream_t s, char **dev);
+  int reserve(Staging &st, size_t bytes);
+  int put(Staging &st, const void *data, size_t bytes, hipStream_t s, char **dev);
 
 private:
   struct Slot {
     char *host = nullptr, *dev = nullptr;
     size_t cap = 0;
     hipEvent_t used = nullptr; // recorded behind the slot's users
-  } slot_[4];
+  } slot_[SLOTS];
   int cur_ = -1;
 };
 
 class BatchEngine {
 public:
   ~BatchEngine();
-  int init(hipStream_t s, const ubg_params &prm, int vcycles_per_step);
+  // members: how many domains to have tables for at once (more are allocated
+  // when they come)
+  int init(hipStream_t s, const ubg_params &prm, int vcycles_per_step, int members);
   hipStream_t stream() const { return stream_; }
   const ubg_params &params() const { return prm_; }
   int vcycles() const { return k_; }
@@ -212,6 +239,7 @@ private:
     size_t off;
   };
   int build_tables();
+  int reserve_active(size_t n);
   int build_tiles();
   void gen_steps(int nsteps, std::vector<StageRec> &st, std::vector<uint8_t> &idx,
                  bool all_fresh = false);
@@ -228,6 +256,7 @@ private:
   std::vector<BDomain *> run_, fresh_, all_;
   int lmax_ = 0;
   // device tables
+  Staging staging_;
   UploadRing tab_ring_, off_ring_, idx_ring_, st_ring_;
   BLev *d_lev_ = nullptr; // in tab_ring_, as are d_dom_ and d_cargs_
   BDom *d_dom_ = nullptr;

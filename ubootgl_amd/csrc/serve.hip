@@ -46,6 +46,9 @@ struct SrvReq {
 
 } // namespace
 
+// domains in a step that a new server has tables for
+constexpr int kMembers = 64;
+
 struct ubg_server {
   ubg_server_params prm{};
   ubg::BatchEngine eng;
@@ -297,7 +300,7 @@ UBG_API int ubg_server_create(const ubg_server_params *prm, const ubg_params *mg
     return fail(UBG_E_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
   int rc = S->arena.init(P.hbm_budget);
-  if (rc == UBG_OK) rc = S->eng.init(S->stream, M, P.vcycles_per_iter);
+  if (rc == UBG_OK) rc = S->eng.init(S->stream, M, P.vcycles_per_iter, std::min(P.max_active, kMembers));
   if (rc != UBG_OK) {
     S->arena.release();
     (void)hipStreamDestroy(S->stream);
