@@ -783,6 +783,7 @@ int BatchEngine::domain_read_state(BDomain *d, DState *out, hipStream_t s) {
 int BatchEngine::start_all(const std::vector<BDomain *> &doms, double tol, int max_iter) {
   const size_t n = doms.size(), ptr_bytes = al(n * sizeof(DState *));
   if (!n) return UBG_OK;
+  if (n == 1) return domain_start(doms[0], tol, max_iter); // one copy instead of a table and a launch
   std::vector<char> blob(states_bytes(n));
   for (size_t i = 0; i < n; i++) {
     ((DState **)blob.data())[i] = doms[i]->st;
@@ -800,6 +801,7 @@ int BatchEngine::read_states(const std::vector<BDomain *> &doms, std::vector<DSt
   const size_t n = doms.size(), ptr_bytes = al(n * sizeof(DState *));
   out.resize(n);
   if (!n) return UBG_OK;
+  if (n == 1) return domain_read_state(doms[0], out.data());
   std::vector<char> blob(states_bytes(n));
   for (size_t i = 0; i < n; i++) ((DState **)blob.data())[i] = doms[i]->st;
   char *dev = nullptr;
@@ -1255,56 +1257,79 @@ std::string BatchEngine::state_key() const {
   return k;
 }
 
+// The stages that `gen` makes, as a captured graph per index state and `what`
+// (their index rows in a device buffer of the graph's own), replayed
+template <class Gen> int BatchEngine::replay(const std::string &what, Gen gen) {
+  const std::string key = state_key() + what;
+  std::vector<std::array<int, BMAXL + 1>> start;
+  for (BDomain *d : all_) {
+    std::array<int, BMAXL + 1> c;
+    std::copy(d->cur, d->cur + BMAXL, c.begin());
+    c[BMAXL] = d->xcur;
+    start.push_back(c);
+  }
+  // the host index state moves on as the schedule does, unless it cannot run
+  std::vector<StageRec> st;
+  std::vector<uint8_t> idx;
+  gen(st, idx);
+  auto undo = [&] {
+    for (size_t i = 0; i < all_.size(); i++) {
+      std::copy(start[i].begin(), start[i].end() - 1, all_[i]->cur);
+      all_[i]->xcur = start[i][BMAXL];
+    }
+  };
+  auto it = graphs_.find(key);
+  if (it == graphs_.end()) {
+    Graph g;
+    const int rc = capture(st, idx, &g);
+    if (rc != UBG_OK) {
+      undo();
+      return rc;
+    }
+    it = graphs_.emplace(key, g).first;
+  }
+  const hipError_t e = hipGraphLaunch(it->second.exec, stream_);
+  if (e != hipSuccess) undo();
+  UBG_HIP(e);
+  return UBG_OK;
+}
+
+int BatchEngine::capture(const std::vector<StageRec> &st, const std::vector<uint8_t> &idx,
+                         Graph *g) {
+  UBG_HIP(hipMalloc((void **)&g->d_idx, std::max<size_t>(idx.size(), 1)));
+  hipError_t e = hipMemcpy(g->d_idx, idx.data(), idx.size(), hipMemcpyHostToDevice);
+  hipGraph_t graph = nullptr;
+  int rc = UBG_OK;
+  if (e == hipSuccess) e = hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal);
+  if (e == hipSuccess) {
+    rc = launch_stages(st, g->d_idx);
+    e = hipStreamEndCapture(stream_, &graph);
+  }
+  if (rc == UBG_OK && e == hipSuccess) e = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
+  if (graph) (void)hipGraphDestroy(graph);
+  if (rc == UBG_OK && e == hipSuccess) return UBG_OK;
+  (void)hipFree(g->d_idx);
+  return rc != UBG_OK ? rc : fail(UBG_E_HIP, std::string("graph capture: ") + hipGetErrorString(e));
+}
+
+int BatchEngine::replay_steps(int nsteps) {
+  if (!fresh_.empty()) return fail(UBG_E_STATE, "graph replay needs every member running");
+  return replay("/" + std::to_string(nsteps),
+                [&](std::vector<StageRec> &st, std::vector<uint8_t> &idx) { gen_steps(nsteps, st, idx); });
+}
+
 int BatchEngine::enqueue_vcycles(int ncycles, bool zg) {
   if (!tiled() || prm_.nu_pre < 1 || prm_.nu_post < 1)
     return fail(UBG_E_INVALID, "projection batches need 1..3 pre- and post-smoothing sweeps");
   if (!fresh_.empty()) return fail(UBG_E_STATE, "projection batches take running members only");
   if (run_.empty() || ncycles <= 0) return UBG_OK;
-  // one captured graph per index state (the V-cycles of all members, their
-  // index rows in a device buffer of the graph's own), replayed
-  const std::string key =
-      state_key() + "/v" + std::to_string(ncycles) + (zg ? "z" : "n");
-  auto it = graphs_.find(key);
-  if (it == graphs_.end()) {
-    std::vector<std::array<int, BMAXL>> saved;
-    for (BDomain *d : all_) {
-      std::array<int, BMAXL> c;
-      for (int l = 0; l < BMAXL; l++) c[l] = d->cur[l];
-      saved.push_back(c);
-    }
-    std::vector<StageRec> st;
-    std::vector<uint8_t> idx;
-    for (int v = 0; v < ncycles; v++) gen_vcycle_tiled(st, idx);
-    for (size_t i = 0; i < all_.size(); i++)
-      for (int l = 0; l < BMAXL; l++) all_[i]->cur[l] = saved[i][l];
-    Graph g;
-    UBG_HIP(hipMalloc((void **)&g.d_idx, std::max<size_t>(idx.size(), 1)));
-    UBG_HIP(hipMemcpy(g.d_idx, idx.data(), idx.size(), hipMemcpyHostToDevice));
-    hipGraph_t graph = nullptr;
-    UBG_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    zg0_ = zg;
-    int rc = launch_stages(st, g.d_idx);
-    zg0_ = false;
-    hipError_t e = hipStreamEndCapture(stream_, &graph);
-    if (rc != UBG_OK || e != hipSuccess) {
-      if (graph) (void)hipGraphDestroy(graph);
-      (void)hipFree(g.d_idx);
-      return rc != UBG_OK ? rc : fail(UBG_E_HIP, std::string("graph capture: ") + hipGetErrorString(e));
-    }
-    e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    if (e != hipSuccess) {
-      (void)hipFree(g.d_idx);
-      return fail(UBG_E_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
-    }
-    it = graphs_.emplace(key, g).first;
-  }
-  UBG_HIP(hipGraphLaunch(it->second.exec, stream_));
-  // advance the host index state as the schedule does
-  std::vector<StageRec> st;
-  std::vector<uint8_t> idx;
-  for (int v = 0; v < ncycles; v++) gen_vcycle_tiled(st, idx);
-  return UBG_OK;
+  zg0_ = zg;
+  const int rc = replay("/v" + std::to_string(ncycles) + (zg ? "z" : "n"),
+                        [&](std::vector<StageRec> &st, std::vector<uint8_t> &idx) {
+                          for (int v = 0; v < ncycles; v++) gen_vcycle_tiled(st, idx);
+                        });
+  zg0_ = false;
+  return rc;
 }
 
 std::vector<BDomain *> BatchEngine::active_members() const {
@@ -1905,12 +1930,17 @@ UBG_API int ubg_batch_solve(ubg_batch *b, const ubg_ir_params *prm, int *graph_r
   // and instantiated per member set, over tables copied with two
   // synchronisations, left the GPU idle meanwhile: 24 domains of 128 to 1024
   // cells a side 10.1 -> 7.9 ms, 60 of 100x90 to 513x385 14.4 -> 10.2 ms, one
-  // domain the same (256x200: 2.73 and 2.75 ms).
+  // domain the same (256x200: 2.73 and 2.75 ms).  Only a batch of one domain with
+  // a launch per sweep runs its launches faster than they are enqueued, and its
+  // member set stays: replayed (64x64 at 20 sweeps 1.83 -> 1.69 ms, 256x200 6.2
+  // -> 5.5; two domains of 48x48 the other way round, 2.7 and 3.7, for a graph
+  // of the one that is left).
+  const bool lone_sweeps = b->doms.size() == 1 && !b->eng.tiled();
   int rounds = 0;
   while (b->eng.active_count() > 0 && 2 * rounds < P.max_iter + 2) {
     std::vector<ubg::BDomain *> act = b->eng.active_members();
     if (act.size() != b->eng.members()) UBG_TRY(b->eng.set_members(act, {}));
-    UBG_TRY(b->eng.enqueue_steps(2));
+    UBG_TRY(lone_sweeps ? b->eng.replay_steps(2) : b->eng.enqueue_steps(2));
     UBG_TRY(b->eng.sync());
     rounds++;
   }

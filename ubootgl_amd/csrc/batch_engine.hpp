@@ -165,6 +165,8 @@ public:
   hipStream_t stream() const { return stream_; }
   const ubg_params &params() const { return prm_; }
   int vcycles() const { return k_; }
+  // levels run as the pre / post passes (smoothing counts that they take)
+  bool tiled() const { return prm_.nu_pre <= kNuPass && prm_.nu_post <= kNuPass; }
   void set_vcycles(int k) {
     if (k != k_) drop_graphs();
     k_ = k;
@@ -214,6 +216,8 @@ public:
   // enqueue `nsteps` refinement steps of the members; the active-domain
   // count lands in *count_host (pinned) when the stream reaches it
   int enqueue_steps(int nsteps);
+  // the same from a captured graph (no fresh members)
+  int replay_steps(int nsteps);
   // the first update (r0, no V-cycles) of every member, as if all were fresh
   int enqueue_first_update();
   // ncycles plain FP32 V-cycles (MG::solve, pressure_solver.cpp:250-257) of
@@ -278,19 +282,19 @@ private:
   Span sw_[BMAXL], rr_[BMAXL], pc_[BMAXL], upd_;
   Span tp_[BMAXL], tq_[BMAXL]; // level passes (pre, post)
   bool zg0_ = false;            // the stages being launched apply ZG at level 0
-  // levels run as the pre / post passes (smoothing counts that they take)
-  bool tiled() const { return prm_.nu_pre <= kNuPass && prm_.nu_post <= kNuPass; }
   int launch_passes_only(int reps);
   int *d_count_ = nullptr;
   int *count_host_ = nullptr;
   uint8_t *d_active_ = nullptr; // per slot, written with the count
   uint8_t *h_active_ = nullptr; // pinned copy
-  // graphs by index state (projection batches with a fixed member set)
+  // graphs by index state (member sets that stay: projection batches, lone domains)
   struct Graph {
     hipGraphExec_t exec = nullptr;
     uint8_t *d_idx = nullptr;
   };
   std::map<std::string, Graph> graphs_;
+  template <class Gen> int replay(const std::string &what, Gen gen);
+  int capture(const std::vector<StageRec> &st, const std::vector<uint8_t> &idx, Graph *g);
   void drop_graphs();
 };
 
