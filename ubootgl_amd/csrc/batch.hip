@@ -681,6 +681,7 @@ int BatchEngine::domain_create(Arena &arena, BGeom *g, float h, BDomain **out, h
   BShape sh;
   UBG_TRY(batch_shape(g->W, g->H, &sh));
   auto *d = new BDomain();
+  d->id = next_id_++;
   d->g = g;
   d->h = h;
   d->bytes = sh.dom_bytes;
@@ -857,11 +858,16 @@ void BatchEngine::drop_graphs() {
 
 int BatchEngine::set_members(const std::vector<BDomain *> &running,
                              const std::vector<BDomain *> &fresh) {
-  if (running == run_ && fresh == fresh_ && d_lev_) return UBG_OK;
+  // by their ids: a released member's address may be another domain's by now
+  std::vector<uint64_t> ids;
+  for (const auto *v : {&running, &fresh})
+    for (const BDomain *d : *v) ids.push_back(d->id);
+  if (ids == ids_ && running.size() == run_.size() && d_lev_) return UBG_OK;
   run_ = running;
   fresh_ = fresh;
   all_ = running;
   all_.insert(all_.end(), fresh.begin(), fresh.end());
+  ids_ = std::move(ids);
   drop_graphs();
   int rc = build_tables();
   if (rc == UBG_OK) rc = build_tiles();

@@ -83,6 +83,7 @@ struct BGeom {
 };
 
 struct BDomain {
+  uint64_t id = 0; // no two domains of an engine have the same
   BGeom *g = nullptr;
   float h = 0.0f;
   float hh[BMAXL] = {};
@@ -203,13 +204,13 @@ public:
   // the member set of the following steps: `running` domains take V-cycles
   // and an accumulating update; `fresh` ones only their first update
   int set_members(const std::vector<BDomain *> &running, const std::vector<BDomain *> &fresh);
-  // forget the member set (a member domain was replaced: a new domain may
-  // sit at the old one's address with other buffers; or its tables could not
-  // be built), so the next set_members rebuilds the tables
+  // forget the member set (a member domain is about to be released, or the
+  // tables could not be built), so the next set_members rebuilds the tables
   void invalidate_members() {
     run_.clear();
     fresh_.clear();
     all_.clear();
+    ids_.clear();
     d_lev_ = nullptr;
     drop_graphs();
   }
@@ -258,6 +259,8 @@ private:
   int k_ = 4;
   Tuning tune_{};
   std::vector<BDomain *> run_, fresh_, all_;
+  std::vector<uint64_t> ids_; // of all_, when the tables were built
+  uint64_t next_id_ = 1;
   int lmax_ = 0;
   // device tables
   Staging staging_;
