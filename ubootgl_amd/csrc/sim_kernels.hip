@@ -183,7 +183,9 @@ __device__ __forceinline__ float fbit(unsigned m, int k) { return ((m >> k) & 1u
 // Blocks go round-robin over the 8 XCDs, so in launch order the rows above and
 // below a block's are read through other L2s.  Diffuse and correction with one
 // cell a lane give each XCD one eighth of the grid in a piece: 1090x436 7.4 ->
-// 5.6 and 6.5 -> 5.5 us, 1921x1081 12.0 -> 12.2 and 13.9 -> 12.3.  (Divergence,
+// 5.6 and 6.5 -> 5.5 us, 1921x1081 12.0 -> 12.2 and 13.9 -> 12.3.  On fields one
+// block wide all passes together, 255x5000 71 -> 64 us, but 160x60000 454 -> 468.
+// (Divergence,
 // which reads each value at most twice, and advect, bound by arithmetic, keep
 // the launch order: no gain, and 1 - 2 us more for a 1921x1081 step.)
 struct BlockXY {
@@ -1221,21 +1223,41 @@ void launch_set_vbcs_vy(const VelView &v, const BCs &bc, hipStream_t s) {
 void launch_face_masks(const uint8_t *flag, uint16_t *fmask, int W, int H, hipStream_t s) {
   hipLaunchKernelGGL(k_face_masks, dim3(ceil_div(W, TPB), H), dim3(TPB), 0, s, flag, fmask, W, H);
 }
-// Whether a pass takes wide rows, and its grid.  One cell a lane is the faster
-// form while the fields stay in the 256 MB last-level cache, two cells a lane
-// where they come from memory, the sooner the more a pass is loads and stores
-// (us, one cell / two): divergence from 2.5M cells (2.1M 10.3 / 10.2, 3.4M
-// 14.2 / 12.0, 8.4M 28.9 / 22.0, 33.6M 125 / 87), correction from 5M (4.5M
-// 22.3 / 24.4, 6.0M 32.3 / 31.3, 8.4M 51 / 45, 33.6M 184 / 170), diffuse
-// beyond 9M (6.0M 27 / 30, 8.4M 39.6 / 40.8, 33.6M 184 / 131; one row a wave
-// instead of two: 146).
-enum WidePass { WIDE_FROM_DIVERGENCE = 2500000, WIDE_FROM_CORRECT = 5000000, WIDE_FROM_DIFFUSE = 9000000 };
-static bool wide_rows(int W, int H, WidePass from, int rows, dim3 *grid) {
-  const bool wide = (long)W * H >= from;
-  const unsigned band = 8 * WIDE_BAND;
-  *grid = wide ? dim3(ceil_div(W - 1, WIDE),
-                      ceil_div(ceil_div(H - 2, WIDE_WAVES * rows), band) * band)
-               : dim3(ceil_div(W - 2, TPB), H - 2);
+// Whether a pass takes wide rows, and its grid.
+//
+// By cells: one cell a lane is the faster form while the fields stay in the 256
+// MB last-level cache, two cells a lane where they come from memory, the sooner
+// the more a pass is loads and stores (us, one cell / two): divergence from
+// 2.5M cells (2.1M 10.3 / 10.2, 3.4M 14.2 / 12.0, 8.4M 28.9 / 22.0, 33.6M 125 /
+// 87), correction from 5M (4.5M 22.3 / 24.4, 6.0M 32.3 / 31.3, 8.4M 51 / 45,
+// 33.6M 184 / 170), diffuse beyond 9M (6.0M 27 / 30, 8.4M 39.6 / 40.8, 33.6M
+// 184 / 131; one row a wave instead of two: 146).
+//
+// By strips: a field a few strips wide leaves lanes of the last one idle, and
+// with 4, 8 or 12 of them blocks above one another meet in the same L2 channels.
+// Divergence and correction from 9 strips but 12 (us, one / two: 130x65000 50 /
+// 92 and 94 / 142, 420x40000 74 / 118 and 129 / 186, 500x40000 85 / 111 and 129 /
+// 162, 870x9700 32 / 40 and 63 / 68, 1000x20000 83 / 76 and 120 / 120, 1100x15000
+// 62 / 58 and 101 / 95; 1478 wide, 12 strips, 2 and 5 longer at 16.4M cells, 1602
+// wide 6 and 9 shorter), diffuse from 5 (255x60000 110 / 124, 420x40000 123 / 137,
+// 500x40000 140 / 132, 1000x20000 134 / 105; 12 strips 10 shorter).
+//
+// By rows: the blocks are rounded up to whole bands on all XCDs, and with few
+// bands some XCDs have one more than others (28000x560, an eighth more rows: 81 /
+// 94 in the correction; 65000x160, 60% more: diffuse 52 / 64, correction 58 / 83).
+struct WidePass {
+  long cells;      // from
+  unsigned strips, not_strips; // from, except
+  int extra;       // rows that the rounding may add, in eighths
+};
+constexpr WidePass WIDE_DIVERGENCE{2500000, 9, 12, 1}, WIDE_CORRECT{5000000, 9, 12, 1},
+    WIDE_DIFFUSION{9000000, 5, 0, 3};
+static bool wide_rows(int W, int H, const WidePass &from, int rows, dim3 *grid) {
+  const unsigned strips = ceil_div(W - 1, WIDE), need = ceil_div(H - 2, WIDE_WAVES * rows);
+  const unsigned blocks = ceil_div(need, 8 * WIDE_BAND) * (8 * WIDE_BAND);
+  const bool wide = (long)W * H >= from.cells && strips >= from.strips && strips != from.not_strips &&
+                    8ul * (blocks - need) <= (unsigned long)from.extra * need;
+  *grid = wide ? dim3(strips, blocks) : dim3(ceil_div(W - 2, TPB), H - 2);
   return wide;
 }
 void launch_diffuse_both(const VelView &v, const uint16_t *fmask, float a, const BCs &bc,
@@ -1243,7 +1265,7 @@ void launch_diffuse_both(const VelView &v, const uint16_t *fmask, float a, const
   BCGrid gx{v.vxb, v.vxf, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyb, v.vyf, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
   dim3 grid;
-  auto k = wide_rows(v.W, v.H, WIDE_FROM_DIFFUSE, WIDE_DIFFUSE, &grid) ? k_diffuse_wide
+  auto k = wide_rows(v.W, v.H, WIDE_DIFFUSION, WIDE_DIFFUSE, &grid) ? k_diffuse_wide
                                                                        : k_diffuse_both;
   hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vxb, v.vyf, v.vyb, fmask, v.W, v.H, a, gx,
                      gy);
@@ -1252,7 +1274,7 @@ void launch_vbcs_divergence(const VelView &v, const BCs &bc, float *f, float ih,
   BCGrid gx{v.vxf, v.vxb, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyf, v.vyb, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
   dim3 grid;
-  auto k = wide_rows(v.W, v.H, WIDE_FROM_DIVERGENCE, 1, &grid) ? k_vbcs_divergence_wide
+  auto k = wide_rows(v.W, v.H, WIDE_DIVERGENCE, 1, &grid) ? k_vbcs_divergence_wide
                                                                : k_vbcs_divergence;
   hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vyf, f, v.W, v.H, ih, gx, gy);
 }
@@ -1261,7 +1283,7 @@ void launch_correct_tail(const VelView &v, float *p, const uint16_t *fmask, floa
   BCGrid gx{v.vxf, v.vxb, v.W - 1, v.H, bc.west, bc.east, bc.south, bc.north, true};
   BCGrid gy{v.vyf, v.vyb, v.W, v.H - 1, bc.west, bc.east, bc.south, bc.north, false};
   dim3 grid;
-  auto k = wide_rows(v.W, v.H, WIDE_FROM_CORRECT, 1, &grid) ? k_correct_tail_wide : k_correct_tail;
+  auto k = wide_rows(v.W, v.H, WIDE_CORRECT, 1, &grid) ? k_correct_tail_wide : k_correct_tail;
   hipLaunchKernelGGL(k, grid, dim3(TPB), 0, s, v.vxf, v.vyf, p, fmask, v.W, v.H, ih, gx, gy, xcur,
                      ycur, bc.west, bc.east, bc.north, bc.south);
 }
