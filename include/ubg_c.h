@@ -219,7 +219,8 @@ UBG_API int ubg_mg_ir_device_ptrs(ubg_mg *mg, double **x, float **f);
  * (sweeps, residual+restriction, prolongation+correction; the coarse levels
  * of each domain in one LDS workgroup), and the refinement steps of all
  * domains (V-cycles, FP64 update, per-domain norm and convergence test) are
- * enqueued two at a time; a converged domain drops out on the device.  Each
+ * enqueued two at a time (a batch of one domain with a launch per sweep replays
+ * them as a captured hipGraph); a converged domain drops out on the device.  Each
  * domain's result is bit-identical to ubg_mg_ir_solve on that domain alone.
  * Domains need W, H >= 16. */
 typedef struct ubg_batch ubg_batch;

@@ -428,7 +428,8 @@ __device__ __forceinline__ void lds_top(const CoarseArgs &a, char *smem, const f
 // solution is written to p0.  A first level of more than kCoarseMaxCells
 // cells is taken only where no smaller one exists (very elongated domains),
 // so it is the coarsest level too: BIG, a variant of its own because it needs
-// more registers.
+// more registers (all 128 that 1024 threads have, and five in scratch, against
+// 118).
 template <bool BIG>
 __device__ __forceinline__ void coarse_vcycle_body(const CoarseArgs &a, const float *f0,
                                                   float *p0) {

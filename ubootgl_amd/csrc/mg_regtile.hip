@@ -54,10 +54,16 @@ long tiles(const Level &L, PassShape shape, bool pre, int nu) {
 }
 // fn(the level's RegTile).  Beyond the shapes of pass_shape: three sweeps on
 // more than 32 tiles per CU take 12 waves of 6 rows, whose halo is an even
-// smaller share (8192x4096 under the zero-gradient BC 143 + 131 us against 158
-// + 133 with 8 waves, without it 129 + 114 against 158 + 125; 4096x2048 41.0 +
-// 38.6 against 41.4 + 39.4, 2048x1024 18.5 + 18.4 against 17.4 + 17.3; with
-// two sweeps the post pass loses, 126 against 118 at 8192x4096).
+// smaller share.  Both compiled for 6 waves a SIMD, pre + post in us with 12
+// waves against 8, under the zero-gradient BC and without it:
+//   8192x4096  152 + 138 against 168 + 144    147 + 133 against 162 + 132
+//   6144x3072   77 +  79 against  83 +  82     73 +  76 against  78 +  74
+//   4096x2048   41 +  39 against  42 +  40     37 +  35 against  39 +  37
+//   3072x1536   30 +  27 against  29 +  28     27 +  25 against  27 +  25
+//   2048x1024   19 +  18 against  18 +  18     16 +  17 against  16 +  17
+// 4096x2048 (18 tiles per CU) stays with 8: a whole step (627 us) and a whole
+// solve (8.73 ms) there take the same with either, within 0.5%.  With two sweeps the post pass loses, 129
+// against 122 at 8192x4096, and the pre pass gains as much.
 template <class Fn> void with_level(const Level &L, bool pre, int nu, Fn fn) {
   const long small = tiles(L, PASS_SMALL, pre, nu);
   if (nu == 3 && small > 32 * kPassCUs) fn(RegTile<3, 6, 12>{});

@@ -10,10 +10,13 @@
 // Each GPU holds its own copy of `scratch` until the process ends, at its own
 // address: the address is looked up with hipGetSymbolAddress once per device
 // (first call with that device current) and only that address is passed to
-// kernels.  All calls on one GPU share the array and every call clears the
-// part it uses first, so a call's result does not depend on earlier calls;
-// calls that overlap on one GPU (other streams, other host threads) race on
-// it and must be ordered by the caller.
+// kernels.  All calls on one GPU share the array.  A call's result does not
+// depend on earlier calls: flags and masks are written and the coarse fields
+// cleared first, and the level-0 second buffer, which holds what the last call
+// left there, is written whole (ring and corners included) by the first sweep
+// or level pass, before anything reads it.  Calls that overlap on one GPU (other
+// streams, other host threads) race on the array and must be ordered by the
+// caller.
 #include "capi_common.hpp"
 
 namespace ubg {
@@ -115,7 +118,7 @@ extern "C" UBG_API int ubg_mg_solve_device_noalloc(float *p, const float *f, con
     L.mask = (uint8_t *)take(n);
   }
   // a fresh hierarchy: the flags, masks and coarse classification, and zero
-  // coarse fields (level 0's second buffer is written whole before it is read)
+  // coarse fields
   m.flag_gen++;
   launch_classify(m.lv.data(), nl, flag, true, s);
   const size_t n0 = (size_t)width * height;

@@ -100,8 +100,11 @@ template <int NU_, int RPW_, int WAVES_> struct RegTile {
   // waves per SIMD to compile the single-domain passes for: with 6 rows, three
   // workgroups of 8 waves or two of 12 a CU need 6 (82 registers instead of 80
   // leave one less: pre without the zero-gradient BC 39.9 instead of 34.5 us at
-  // 4096x2048, 189 instead of 129 with 12 waves at 8192x4096).  The batched
-  // passes spill under that bound (24.9 us instead of 22.9) and keep 4.
+  // 4096x2048, 189 instead of 129 with 12 waves at 8192x4096).  Without the
+  // zero-gradient BC pre reaches 80 (at two and three sweeps) by keeping two of
+  // them in scratch, 12 bytes a lane, which those times include; with it pre
+  // needs 79, post 66.  The batched passes, which also walk their
+  // tiles, spill more under that bound (24.9 us instead of 22.9) and keep 4.
   static constexpr int MINW = RPW >= 6 ? 6 : 4;
   static_assert(RPW % 2 == 0, "a register's colour does not depend on the wave");
   // pre: residuals on [X0-1, X0+otx-1] read p on [X0-2, X0+otx]; each sweep
@@ -357,8 +360,8 @@ template <class T> struct TileRegs {
     }
   }
   // publish / fetch the cells of colour S in the wave's first and last row;
-  // a buffer is written again two exchanges later, when every wave has
-  // passed the barrier after its reads
+  // a buffer is written again three exchanges later, when every wave has
+  // passed the barriers after its reads
   __device__ __forceinline__ float *slot(int buf, int v, int last) const {
     return xb + buf * T::XBUF + (v * 2 + last) * T::XROW + lane;
   }

@@ -84,15 +84,16 @@ void launch_build_mask(const uint8_t *flag, uint8_t *mask, int w, int h, hipStre
 // from; zero: p, p_alt and f of the coarse levels are cleared
 void launch_classify(const Level *lv, int levels, const uint8_t *raw, bool zero, hipStream_t s);
 // one red+black sweep fused in one launch (streaming waves, ping-pong: reads
-// L.p, writes L.p_alt, then swaps the two pointers); zero_gradient applies
-// setZeroGradientBC to the result.
+// L.p, writes all of L.p_alt, ring and corners included, then swaps the two
+// pointers); zero_gradient applies setZeroGradientBC to the result.
 void launch_rbgs_fused(Level &L, float h, float alpha, bool zero_gradient, hipStream_t s);
 void launch_zero_gradient(float *p, int w, int h, hipStream_t s);
-// Level passes (mg_regtile.hip; ping-pong: read L.p, write L.p_alt, swap) of
-// up to kNuPass sweeps:
+// Level passes (mg_regtile.hip; ping-pong: read L.p, write all of L.p_alt, ring
+// and corners included, swap) of up to kNuPass sweeps:
 //   nu sweeps, residual, restriction into C.  zero_p: L.p is zero on entry
-//   and is not read (below the finest level: zg is not looked at); zero_coarse: C.p = 0 in the interior (else C.p is left
-//   as it is, for a coarse pass that does not read it);
+//   and is not read (below the finest level: zg is not looked at);
+//   zero_coarse: C.p = 0 in the interior (else C.p is left as it is, for a
+//   coarse pass that does not read it);
 constexpr int kNuPass = 3;
 void launch_level_pre(Level &L, Level &C, int nu, float h, float alpha, bool zero_p, bool zg,
                       bool zero_coarse, hipStream_t s);
